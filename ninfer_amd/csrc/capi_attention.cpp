@@ -192,6 +192,20 @@ struct PromptChunks {
 
 PromptChunks prompt_chunks(int32_t T) { return PromptChunks{T / kAttnMaxTokens, T % kAttnMaxTokens}; }
 
+// Whether the prompt kernel takes the call, instead of verify launches of 32 tokens. It moves 16-byte
+// pieces of q, out and the cache rows, so all of them have to be 16-byte aligned (any tensor from an
+// allocator is; the verify launches take the rest). At head_dim 128 two launches of the 80-row verify
+// form still serve up to 64 tokens (43 us over 2,048 rows of history). At head_dim 256 those launches take
+// 32-row chunks that each stream every key, and the prompt kernel is ahead from 33 tokens (24/4 heads, 64
+// tokens, 2,048 rows: 53 -> 33 us) until the history is so long that few row tiles cannot split it far
+// enough (33 tokens over 8,000 rows: 53 us by launches, 55 us here).
+bool prompt_kernel_serves(const AttnShape& s, const CacheRef& c, const nmi_tensor* q, const nmi_tensor* out,
+                          uint32_t max_keys) {
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    if (c.kb == nullptr && !(aligned(c.kc) && aligned(c.vc) && aligned(c.ks) && aligned(c.vs))) { return false; }
+    return aligned(q->data) && aligned(out->data) && (s.T > 64 || (s.D == 256 && max_keys <= 4096));
+}
+
 // static_ws: the split partials go to the device's static scratch (the allocation-free entry
 // point); ws/ws_bytes are then ignored.
 int attention_impl(const nmi_tensor* q, const nmi_tensor* k, const nmi_tensor* v,
@@ -233,6 +247,11 @@ int attention_impl(const nmi_tensor* q, const nmi_tensor* k, const nmi_tensor* v
             if (write_cache) {
                 launch_kv_append(static_cast<const uint16_t*>(k->data), static_cast<const uint16_t*>(v->data),
                                  static_cast<const int32_t*>(positions->data), nullptr, CommitBounds{}, s.T, c, stream);
+            }
+            if (prompt_kernel_serves(s, c, q, out, env.max_visible_keys)) {
+                launch_prompt_attention(static_cast<const uint16_t*>(q->data), static_cast<const int32_t*>(positions->data),
+                                        s.T, s.Hq, c, scale, env.max_visible_keys, ws, need, out->data, s.out_f32, stream);
+                return;
             }
             const size_t out_elem = s.out_f32 ? 4 : 2;
             for (int32_t t0 = 0; t0 < s.T; t0 += kAttnMaxTokens) {

@@ -97,6 +97,12 @@ void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uin
                              void* workspace, const SplitPlan& plan, void* out, bool out_f32,
                              hipStream_t stream);
 
+// Causal attention of one sequence's T prompt tokens over cache rows that hold them already
+// (prompt_attention.hip). Key splits' partials go to the workspace, as many as fit.
+void launch_prompt_attention(const uint16_t* q, const int32_t* positions, int32_t T, int32_t Hq, const CacheRef& cache,
+                             float scale, uint32_t max_keys, void* workspace, size_t workspace_bytes, void* out,
+                             bool out_f32, hipStream_t stream);
+
 // Commit helpers (kv_commit.hip).
 void launch_kv_rollback(const int32_t* positions, const int32_t* keep_count, int32_t T,
                         const CacheRef& cache, hipStream_t stream);

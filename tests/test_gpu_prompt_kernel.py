@@ -1,0 +1,82 @@
+"""The prompt kernel (A1/A3 above the verify extents) at the edges of its tiles, against the FP64 oracle
+at the verify bars: row tiles of 64, 128 and 256 rows (WK = 4, 2, 1), key tiles of 128 (head_dim 128)
+and 64 keys (256), unsplit and split over the keys; the exact recompute of groups beyond FP16's
+range in both forms; and tensors it cannot address, which the verify launches take."""
+import numpy as np
+import pytest
+
+import ninfer_amd as na
+from ninfer_amd import ops
+from ninfer_amd.device import DeviceArray, DeviceBuffer, synchronize
+from helpers import AttnCase, rel_l2
+import gpu_runner
+
+pytestmark = pytest.mark.gpu
+
+REL_L2_F32 = 1e-3
+
+
+def _run(case, **kw):
+    expected, ref = case.oracle_after_append()
+    out, cache = gpu_runner.run_attention(case, out_f32=True, **kw)
+    for got, want in zip(cache.download(), expected):
+        assert np.array_equal(got, want)
+    err = rel_l2(out, ref)
+    print(f"rel_l2={err:.3e}", flush=True)
+    assert np.all(np.isfinite(out)) and err <= REL_L2_F32, err
+    return out
+
+
+# (heads, D, cache, history, tokens): 5 x 77 = 385 rows end one row past a 64- and 128-row tile; windows one
+# key before, at and past a key tile; one long prompt of 256-row tiles; splits (short prompts over
+# a longer history); a group of one head and one of eight
+@pytest.mark.parametrize("Hq,Hkv,D,kv,L,T", [
+    (40, 8, 128, "i8", 0, 65), (40, 8, 128, "i8", 50, 77), (40, 8, 128, "i8", 51, 77), (40, 8, 128, "i8", 52, 77),
+    (40, 8, 128, "i8", 3000, 66), (40, 8, 128, "i8", 7, 1100), (40, 8, 128, "bf16", 51, 77), (40, 8, 128, "bf16", 2500, 65),
+    (24, 4, 256, "i8", 0, 33), (24, 4, 256, "i8", 31, 33), (24, 4, 256, "i8", 32, 33), (24, 4, 256, "bf16", 2000, 43),
+    (16, 2, 256, "i8", 0, 64), (16, 2, 256, "bf16", 1, 64), (16, 2, 256, "i8", 1500, 129), (24, 4, 256, "i8", 3, 700),
+    (4, 4, 128, "i8", 129, 130), (64, 2, 128, "i8", 10, 70)])
+def test_tile_edges(gpu, Hq, Hkv, D, kv, L, T):
+    print(f"case prompt kernel {Hq}/{Hkv}/{D} {kv} L={L} T={T}", flush=True)
+    _run(AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, kv=kv, seed=6000 + L + T + Hq))
+
+
+# A wide envelope (the plan follows its end, the keys the device positions) and one that clamps them.
+@pytest.mark.parametrize("L,T,cap", [(300, 70, 20000), (700, 300, 40000)])
+def test_wide_envelope(gpu, L, T, cap):
+    print(f"case prompt envelope L={L} T={T} cap={cap}", flush=True)
+    case = AttnCase([L], T=T, seed=61 + T, max_context=cap)
+    _run(case, envelope=(1, cap))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,L,T", [(40, 8, 128, 100, 65), (40, 8, 128, 2600, 65), (24, 4, 256, 150, 40), (24, 4, 256, 1500, 40)])
+@pytest.mark.parametrize("absmax", [1e5, 1e6])
+def test_fp32_range(gpu, Hq, Hkv, D, L, T, absmax):
+    """Scales above 512 in K and V (K' or V' beyond FP16), unsplit and split over the keys: the rows are
+    computed again in FP32, as the verify kernels' merge does. K groups and V groups of their own
+    positions, so rows with only one kind exist."""
+    print(f"case prompt fp32 range {Hq}/{Hkv}/{D} L={L} T={T} absmax={absmax:g}", flush=True)
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, seed=9, qstd=2e-5)
+    rng = np.random.default_rng(5)
+    big = np.float16(absmax / 127.0).view(np.uint16)
+    for sc in (case.ks, case.vs):
+        for _ in range(6):
+            sc[0, int(rng.integers(0, Hkv)), int(rng.integers(0, L)), int(rng.integers(0, D // 64))] = big
+    _run(case)
+
+
+def test_unaligned_tensors_take_the_verify_launches(gpu):
+    """q one element into its buffer: accepted as before, and within the same bar."""
+    case = AttnCase([200], T=70, seed=17)
+    _, ref = case.oracle_after_append()
+    cache = gpu_runner.upload_cache(case)
+    gpu_runner.append(case, cache)
+    D, Hq, T = case.D, case.Hq, case.T
+    raw = DeviceArray.from_numpy(na.BF16, np.concatenate([np.zeros(2, np.uint16), case.q]))
+    q = na.Tensor.make(raw.ptr + 4, na.BF16, (D, Hq, T))
+    pos = DeviceArray.from_numpy(na.I32, case.positions, (T, 1))
+    out = DeviceArray(na.FP32, (D, Hq, T))
+    ws = DeviceBuffer(ops.gqa_attention_workspace_bytes(Hq, case.Hkv, D, T, 1, case.max_context))
+    ops.gqa_attention_cached(q, pos.tensor(), case.scale, cache.view(), (1, case.max_context), ws, out.tensor())
+    synchronize()
+    assert rel_l2(out.numpy().astype(np.float64), ref) <= REL_L2_F32
