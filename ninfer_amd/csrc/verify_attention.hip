@@ -2206,29 +2206,87 @@ __global__ __launch_bounds__(256) void kv_quant_append_kernel(const uint16_t* k,
     }
 }
 
-// BF16 cache append (A2, and A1 on a BF16 cache): column t of sequence b is copied bit for bit into
-// row positions[t] (reference gqa_kv_append on a BF16 cache). Block (t, b, h).
-__global__ __launch_bounds__(64) void bf16_kv_append_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
-                                                            const int32_t* count, CommitBounds cb, int32_t T,
-                                                            int32_t Hkv, int32_t P, int32_t D, uint16_t* kb,
-                                                            uint16_t* vb, int64_t seq) {
-    const int t = blockIdx.x;
-    const int b = blockIdx.y;
-    const int h = blockIdx.z;
+// Column (t, b), KV head and 8-element piece of a flat index over k/v [D, Hkv, T, B] (source offset
+// 8u), and the cache row of the column (-1: the column is not written).
+struct AppendUnit {
+    int piece, h, b, row;
+};
+
+__device__ __forceinline__ AppendUnit append_unit(uint32_t u, uint32_t pieces, const int32_t* positions, const int32_t* count,
+                                                  CommitBounds cb, int32_t T, int32_t Hkv, int32_t P) {
+    AppendUnit x;
+    const uint32_t th = u / pieces;
+    x.piece = static_cast<int>(u - th * pieces);
+    const int col = static_cast<int>(th / static_cast<uint32_t>(Hkv));
+    x.h = static_cast<int>(th - static_cast<uint32_t>(col) * static_cast<uint32_t>(Hkv));
+    x.b = col / T;
+    const int p = positions[col];
+    x.row = p < 0 || (p & cb.slot_mask) >= P ? -1 : p & cb.slot_mask;
     if (count != nullptr) {
-        const int n = count[b];
-        if (n < cb.min_count || n > cb.max_count || t >= n) { return; }
+        const int n = count[x.b];
+        if (n < cb.min_count || n > cb.max_count || col - x.b * T >= n) { x.row = -1; }
     }
-    const int p = positions[static_cast<int64_t>(b) * T + t];
-    if (p < 0) { return; }
-    const int pos = p & cb.slot_mask;
-    if (pos >= P) { return; }
-    const int64_t src = static_cast<int64_t>(D) * (h + static_cast<int64_t>(Hkv) * (t + static_cast<int64_t>(T) * b));
-    const int64_t dst = static_cast<int64_t>(b) * seq + static_cast<int64_t>(D) * (pos + static_cast<int64_t>(P) * h);
-    for (int i = threadIdx.x; i < D / 8; i += blockDim.x) {
-        *reinterpret_cast<i4*>(kb + dst + 8 * i) = *reinterpret_cast<const i4*>(k + src + 8 * i);
-        *reinterpret_cast<i4*>(vb + dst + 8 * i) = *reinterpret_cast<const i4*>(v + src + 8 * i);
+    return x;
+}
+
+// The same encoder over 16-byte aligned k/v and 8-byte aligned code planes: a lane owns 8 consecutive
+// elements, 8 lanes a group, so a wave reads 1 KB and writes 512 B whole. Launch-bound for a verify
+// round's few rows; a 2,048-token prompt of 8 heads (34 MB read and written) took 13.5 us with a wave
+// per 64-element group in 16,384 workgroups of 2-byte loads and 4.1 us this way. y: K or V.
+template <int D>
+__global__ __launch_bounds__(256) void kv_quant_append_rows_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
+                                                                   const int32_t* count, CommitBounds cb, int32_t T, int32_t Hkv,
+                                                                   int32_t P, int8_t* kc, int8_t* vc, uint16_t* ks, uint16_t* vs,
+                                                                   int64_t code_seq, int64_t scale_seq, uint32_t units) {
+    const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+    if (u >= units) { return; } // units is a multiple of 8: whole groups stay together
+    const i4 raw = *reinterpret_cast<const i4*>((blockIdx.y ? v : k) + static_cast<int64_t>(u) * 8);
+    const AppendUnit a = append_unit(u, D / 8, positions, count, cb, T, Hkv, P);
+    float x[8];
+    float amax = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t w = static_cast<uint32_t>(raw[e >> 1]);
+        x[e] = bf16_to_f32(static_cast<uint16_t>((e & 1) ? w >> 16 : w & 0xffffu));
+        amax = fmaxf(amax, fabsf(x[e]));
     }
+    amax = fmaxf(amax, dpp_from<0xB1, 0xf>(amax, 0.0f));  // lane ^ 1
+    amax = fmaxf(amax, dpp_from<0x4E, 0xf>(amax, 0.0f));  // lane ^ 2
+    amax = fmaxf(amax, dpp_from<0x141, 0xf>(amax, 0.0f)); // the other four of the eight
+    const uint16_t sbits = f32_to_f16_bits(amax > 0.0f ? amax / 127.0f : 0.0f);
+    const float s = f16_bits_to_f32(sbits);
+    const float inv = s > 0.0f ? 1.0f / s : 0.0f;
+    uint32_t code[2] = {0u, 0u};
+    if (inv != 0.0f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float rr = rintf(x[e] * inv);
+            rr = fminf(127.0f, fmaxf(-127.0f, rr));
+            code[e >> 2] |= (static_cast<uint32_t>(static_cast<int8_t>(rr)) & 0xffu) << (8 * (e & 3));
+        }
+    }
+    if (a.row < 0) { return; }
+    int8_t* cdst = (blockIdx.y ? vc : kc) + static_cast<int64_t>(a.b) * code_seq + static_cast<int64_t>(D) * (a.row + static_cast<int64_t>(P) * a.h);
+    *reinterpret_cast<i2*>(cdst + 8 * a.piece) = i2{static_cast<int>(code[0]), static_cast<int>(code[1])};
+    if ((a.piece & 7) == 0) {
+        uint16_t* sdst = (blockIdx.y ? vs : ks) + static_cast<int64_t>(a.b) * scale_seq + static_cast<int64_t>(D / 64) * (a.row + static_cast<int64_t>(P) * a.h);
+        sdst[a.piece >> 3] = sbits;
+    }
+}
+
+// BF16 cache append (A2, and A1 on a BF16 cache): column t of sequence b is copied bit for bit into
+// row positions[t] (reference gqa_kv_append on a BF16 cache), 16 bytes per lane. y: K or V.
+__global__ __launch_bounds__(256) void bf16_kv_append_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
+                                                             const int32_t* count, CommitBounds cb, int32_t T,
+                                                             int32_t Hkv, int32_t P, int32_t D, uint16_t* kb,
+                                                             uint16_t* vb, int64_t seq, uint32_t units) {
+    const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+    if (u >= units) { return; }
+    const i4 raw = *reinterpret_cast<const i4*>((blockIdx.y ? v : k) + static_cast<int64_t>(u) * 8);
+    const AppendUnit a = append_unit(u, D / 8, positions, count, cb, T, Hkv, P);
+    if (a.row < 0) { return; }
+    uint16_t* dst = (blockIdx.y ? vb : kb) + static_cast<int64_t>(a.b) * seq + static_cast<int64_t>(D) * (a.row + static_cast<int64_t>(P) * a.h);
+    *reinterpret_cast<i4*>(dst + 8 * a.piece) = raw;
 }
 
 } // namespace
@@ -2352,21 +2410,33 @@ size_t attention_workspace_bound(int32_t Hq, int32_t Hkv, int32_t D, int32_t T) 
 void launch_kv_append(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                       const int32_t* count, CommitBounds bounds, int32_t T, const CacheRef& c,
                       hipStream_t stream) {
-    dim3 grid(T, c.B, c.Hkv);
+    const int64_t units = static_cast<int64_t>(T) * c.B * c.Hkv * (c.D / 8); // 8-element pieces of k
+    if (units > 0xffffff00) { throw Unsupported("kv append: 2^35 or more elements in one call are not built"); }
+    const dim3 flat(static_cast<unsigned>((units + 255) / 256), 2);
     if (c.kb != nullptr) {
-        hipLaunchKernelGGL(bf16_kv_append_kernel, grid, dim3(64), 0, stream, k, v, positions, count, bounds, T, c.Hkv,
-                           c.P, c.D, c.kb, c.vb, c.code_seq);
+        hipLaunchKernelGGL(bf16_kv_append_kernel, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T, c.Hkv,
+                           c.P, c.D, c.kb, c.vb, c.code_seq, static_cast<uint32_t>(units));
         check_launch("bf16_kv_append_kernel");
         return;
     }
-    if (c.D == 128) {
-        hipLaunchKernelGGL(kv_quant_append_kernel<128>, grid, dim3(256), 0, stream, k, v, positions,
-                           count, bounds, T, c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq);
-    } else if (c.D == 256) {
-        hipLaunchKernelGGL(kv_quant_append_kernel<256>, grid, dim3(256), 0, stream, k, v, positions,
-                           count, bounds, T, c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq);
+    const auto misaligned = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
+    if (c.D != 128 && c.D != 256) { throw Unsupported("kv append: head_dim 128 and 256 are built"); }
+    if (misaligned(k, 16) || misaligned(v, 16) || misaligned(c.kc, 8) || misaligned(c.vc, 8)) {
+        // 2-byte loads and 1-byte stores for tensors the wide form cannot address
+        const dim3 grid(T, c.B, c.Hkv);
+        if (c.D == 128) {
+            hipLaunchKernelGGL(kv_quant_append_kernel<128>, grid, dim3(256), 0, stream, k, v, positions,
+                               count, bounds, T, c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq);
+        } else {
+            hipLaunchKernelGGL(kv_quant_append_kernel<256>, grid, dim3(256), 0, stream, k, v, positions,
+                               count, bounds, T, c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq);
+        }
+    } else if (c.D == 128) {
+        hipLaunchKernelGGL(kv_quant_append_rows_kernel<128>, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T,
+                           c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, static_cast<uint32_t>(units));
     } else {
-        throw Unsupported("kv append: head_dim 128 and 256 are built");
+        hipLaunchKernelGGL(kv_quant_append_rows_kernel<256>, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T,
+                           c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, static_cast<uint32_t>(units));
     }
     check_launch("kv_quant_append_kernel");
 }

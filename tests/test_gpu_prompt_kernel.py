@@ -1,7 +1,7 @@
 """The prompt kernel (A1/A3 above the verify extents) at the edges of its tiles, against the FP64 oracle
 at the verify bars: row tiles of 64, 128 and 256 rows (WK = 4, 2, 1), key tiles of 128 (head_dim 128)
 and 64 keys (256), unsplit and split over the keys; the exact recompute of groups beyond FP16's
-range in both forms; and tensors it cannot address, which the verify launches take."""
+range in both forms; tensors it cannot address, which the verify launches take; and the flat append."""
 import numpy as np
 import pytest
 
@@ -80,3 +80,31 @@ def test_unaligned_tensors_take_the_verify_launches(gpu):
     ops.gqa_attention_cached(q, pos.tensor(), case.scale, cache.view(), (1, case.max_context), ws, out.tensor())
     synchronize()
     assert rel_l2(out.numpy().astype(np.float64), ref) <= REL_L2_F32
+
+
+@pytest.mark.parametrize("D,T,B,offset", [(128, 1, 1, 0), (128, 3, 3, 0), (256, 5, 2, 0), (128, 700, 1, 0), (128, 3, 2, 2), (256, 2, 1, 1)])
+def test_append_forms(gpu, D, T, B, offset):
+    """The flat encoder (aligned) and the one-wave-per-group form (`offset` elements off) write the
+    oracle's codes and scales bit for bit, negative positions and zero groups included."""
+    print(f"case append D={D} T={T} B={B} offset={offset}", flush=True)
+    case = AttnCase([10 * (b + 1) for b in range(B)], T=T, Hq=8, Hkv=4, D=D, seed=T + B)
+    case.k_new[:64] = 0
+    case.v_new[64:128] = 0x8000
+    (kc, vc, ks, vs) = (x.copy() for x in case.cache_planes())
+    from oracle import pyoracle
+    pyoracle.kv_append(case.k_new, case.v_new, case.positions, T, B, 4, D, case.P, kc, vc, ks, vs)
+    if T > 1:  # a negative position is skipped (the oracle takes real ones only): its row stays as it was
+        row = int(case.positions[1])
+        for got, was in zip((kc, vc, ks, vs), case.cache_planes()):
+            got[0, :, row] = was[0, :, row]
+        case.positions[1] = -1
+    cache = gpu_runner.upload_cache(case)
+    pad = np.zeros(offset, np.uint16)
+    dk = DeviceArray.from_numpy(na.BF16, np.concatenate([pad, case.k_new]))
+    dv = DeviceArray.from_numpy(na.BF16, np.concatenate([pad, case.v_new]))
+    pos = DeviceArray.from_numpy(na.I32, case.positions, (T, B))
+    ops.gqa_kv_append(na.Tensor.make(dk.ptr + 2 * offset, na.BF16, (D, 4, T, B)),
+                      na.Tensor.make(dv.ptr + 2 * offset, na.BF16, (D, 4, T, B)), pos.tensor(), cache.view())
+    synchronize()
+    for got, want in zip(cache.download(), (kc, vc, ks, vs)):
+        assert np.array_equal(got, want)
