@@ -39,6 +39,10 @@ struct ConvArgs {
     int32_t slots;
 };
 
+// Many tokens at a time (gdn_chunk.hip): whether it takes a call, and its launch.
+bool gdn_chunk_serves(const GdnArgs& a, int32_t S);
+void launch_gdn_chunk(const GdnArgs& a, hipStream_t stream);
+
 void launch_gdn_recurrent(const GdnArgs& a, int32_t S, hipStream_t stream);
 void launch_conv1d_silu(const ConvArgs& a, hipStream_t stream);
 // op: 0 set (dst32 = value), 1 assign (dst32 = *src), 2 increment dst32, 3 increment dst64.

@@ -260,6 +260,10 @@ __global__ void scalar_kernel(int32_t op, const int32_t* src, int32_t* dst32, lo
 } // namespace
 
 void launch_gdn_recurrent(const GdnArgs& a, int32_t S, hipStream_t stream) {
+    if (gdn_chunk_serves(a, S)) {
+        launch_gdn_chunk(a, stream);
+        return;
+    }
     const dim3 grid(S / kGdnRows, a.Hv);
     const dim3 block(kGdnThreads);
     switch (S) {

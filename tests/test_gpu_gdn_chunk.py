@@ -1,0 +1,59 @@
+"""Prompts through the gated delta rule: the chunked form (more than 16 tokens at head dimension 128) at the
+edges of its 32-token chunks, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+from test_gpu_gdn import GDN_OUTPUT_BF16, _f, _inputs, _ok, run_regular
+
+pytestmark = pytest.mark.gpu
+
+# FP32 sums of products exact in FP32, and one BF16 rounding of v's products: the token-by-token kernel
+# is 1.1e-7 to 1.25e-7 from 64 bits in the 2-norm over these ranges, this one 8e-8 to 9e-8.
+STATE_REL = 1.5e-7
+
+
+def _oracle(inp, Hqk, Hv, T, normalize):
+    from oracle import pyoracle
+    return pyoracle.gdn_recurrent(inp["q"], inp["k"], inp["v"], inp["g"], inp["beta"], inp["state"], 128, Hqk, Hv, T, normalize)
+
+
+@pytest.mark.parametrize("T", [17, 31, 32, 33, 63, 64, 65, 97, 130])
+@pytest.mark.parametrize("Hqk,Hv,normalize,in_place", [(16, 48, True, False), (5, 5, True, True), (2, 18, False, False)])
+def test_chunk_edges(gpu, T, Hqk, Hv, normalize, in_place):
+    print(f"case gdn chunk T={T} Hqk={Hqk} Hv={Hv} norm={normalize} in_place={in_place}", flush=True)
+    inp = _inputs(300 + T + Hv, 128, Hqk, Hv, T, normalized=not normalize, stress_g=T % 2 == 1)
+    ref_out, ref_state = _oracle(inp, Hqk, Hv, T, normalize)[:2]
+    out, state = run_regular(inp, 128, Hqk, Hv, T, normalize, in_place)
+    _ok(_f(out).reshape(T, Hv, 128), ref_out, GDN_OUTPUT_BF16, "out")
+    rel = np.linalg.norm(state - ref_state) / np.linalg.norm(ref_state)
+    print(f"state rel {rel:.2e}", flush=True)
+    assert rel <= STATE_REL
+
+
+def test_decay_extremes(gpu):
+    """Decays of exactly 0 and 1, and long runs of strong decay: no difference of logarithms is lost."""
+    T, H = 70, 4
+    inp = _inputs(31, 128, H, H, T, normalized=False)
+    inp["g"][5] = -np.inf
+    inp["g"][6:20] = -0.001
+    inp["g"][20:36] = -90.0
+    inp["g"][36:50] = 0.0
+    ref_out, ref_state = _oracle(inp, H, H, T, True)[:2]
+    out, state = run_regular(inp, 128, H, H, T, True, False)
+    _ok(_f(out).reshape(T, H, 128), ref_out, GDN_OUTPUT_BF16, "out")
+    assert np.linalg.norm(state - ref_state) / np.linalg.norm(ref_state) <= STATE_REL
+
+
+@pytest.mark.parametrize("where", ["v", "k", "q", "g"])
+def test_non_finite_token_leaves_earlier_outputs(gpu, where):
+    """A NaN in token 40 reaches no output before it, as token by token."""
+    T, H = 66, 3
+    inp = _inputs(77, 128, H, H, T, normalized=False)
+    clean = _f(run_regular(inp, 128, H, H, T, True, False)[0]).reshape(T, H, 128)
+    if where == "g":
+        inp["g"][40] = np.nan
+    else:
+        inp[where].reshape(T, H, 128)[40, :, 7] = 0x7FC0
+    out = _f(run_regular(inp, 128, H, H, T, True, False)[0]).reshape(T, H, 128)
+    _ok(out[:40], clean[:40], GDN_OUTPUT_BF16, "out before") # the chunk's products in another order
+    assert np.isnan(out[40]).any()
