@@ -10,6 +10,8 @@
 #include "common.h"
 #include "gdn_internal.h"
 
+#include <initializer_list>
+
 namespace nmi {
 namespace {
 
@@ -246,6 +248,61 @@ __global__ __launch_bounds__(256) void conv1d_silu_kernel(ConvArgs a) {
     }
 }
 
+// The same convolution over a prompt (no snapshots): a thread owns V channels and TILE consecutive tokens,
+// so the chip streams x once instead of walking the tokens in a thread per channel. A tile's window is the
+// state (first tile) or the three tokens before it; the first tile also writes the final window, after
+// reading the one it may replace. 2,000 tokens x 10,240 channels (82 MB read and written) on MI355X: 777 us
+// with a thread per channel, 35 us with 8 x 16 per thread (bound by expf and the division); 33 to 64
+// tokens 13-21 us with a thread per channel, 18 us with 8 x 16 and 6.5 us with 2 x 4 (enough threads).
+template <int V>
+struct ConvVec;
+template <>
+struct ConvVec<1> {
+    uint16_t v[1];
+};
+template <>
+struct alignas(4) ConvVec<2> {
+    uint16_t v[2];
+};
+template <>
+struct alignas(16) ConvVec<8> {
+    uint16_t v[8];
+};
+
+template <int V, int TILE>
+__global__ __launch_bounds__(256) void conv1d_silu_prompt_kernel(ConvArgs a) {
+    using Vec = ConvVec<V>;
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * V;
+    if (c >= a.C) { return; }
+    const int t0 = blockIdx.y * TILE;
+    const auto at = [&](const uint16_t* base, int64_t row) { return *reinterpret_cast<const Vec*>(base + row * a.C + c); };
+    Vec u[3], w[4], x[TILE];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) { u[j] = t0 == 0 ? at(a.state_in, j) : at(a.x, t0 - 3 + j); }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { w[j] = at(a.weight, j); }
+#pragma unroll
+    for (int i = 0; i < TILE; ++i) { x[i] = at(a.x, min(t0 + i, a.T - 1)); }
+#pragma unroll
+    for (int i = 0; i < TILE; ++i) {
+        if (t0 + i >= a.T) { break; }
+        Vec o;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            float acc = bf16_to_f32(w[0].v[e]) * bf16_to_f32(i >= 3 ? x[i - 3].v[e] : u[i].v[e]);
+            acc = fmaf(bf16_to_f32(w[1].v[e]), bf16_to_f32(i >= 2 ? x[i - 2].v[e] : u[i + 1].v[e]), acc);
+            acc = fmaf(bf16_to_f32(w[2].v[e]), bf16_to_f32(i >= 1 ? x[i - 1].v[e] : u[i + 2].v[e]), acc);
+            acc = fmaf(bf16_to_f32(w[3].v[e]), bf16_to_f32(x[i].v[e]), acc);
+            o.v[e] = f32_to_bf16(acc / (1.0f + expf(-acc)));
+        }
+        *reinterpret_cast<Vec*>(a.out + static_cast<int64_t>(t0 + i) * a.C + c) = o;
+    }
+    if (t0 == 0) { // T > 16 here: the last three tokens are x's
+#pragma unroll
+        for (int j = 0; j < 3; ++j) { *reinterpret_cast<Vec*>(a.state_out + static_cast<int64_t>(j) * a.C + c) = at(a.x, a.T - 3 + j); }
+    }
+}
+
 // include/ninfer/ops/scalar.h:27-30.
 __global__ void scalar_kernel(int32_t op, const int32_t* src, int32_t* dst32, long long* dst64, int32_t value) {
     if (threadIdx.x != 0) { return; }
@@ -278,6 +335,33 @@ void launch_gdn_recurrent(const GdnArgs& a, int32_t S, hipStream_t stream) {
 
 void launch_conv1d_silu(const ConvArgs& a, hipStream_t stream) {
     const int threads = 256;
+    if (a.initial_slot == nullptr && a.T > 16) {
+        // pieces of 8 (2) channels where every row of every tensor is 16-byte (4-byte) aligned
+        const auto aligned = [&](uintptr_t n) {
+            for (const void* p : {static_cast<const void*>(a.x), static_cast<const void*>(a.weight), static_cast<const void*>(a.state_in),
+                                  static_cast<const void*>(a.state_out), static_cast<const void*>(a.out)}) {
+                if ((reinterpret_cast<uintptr_t>(p) & (n - 1)) != 0) { return false; }
+            }
+            return a.C % static_cast<int32_t>(n / 2) == 0;
+        };
+        // 8 x 16 values per thread once that still gives 256 CUs two waves per SIMD
+        const bool large = static_cast<int64_t>(a.C) * a.T >= int64_t{8 * 16} * 256 * 512;
+        const int v = large && aligned(16) ? 8 : aligned(4) ? 2 : 1;
+        const int tile = v == 8 ? 16 : 4;
+        const int64_t tiles = (static_cast<int64_t>(a.T) + tile - 1) / tile;
+        if (tiles <= 65535) { // a longer prompt than the grid holds keeps the thread per channel
+            const dim3 grid((a.C + threads * v - 1) / (threads * v), static_cast<unsigned>(tiles));
+            if (v == 8) {
+                hipLaunchKernelGGL((conv1d_silu_prompt_kernel<8, 16>), grid, dim3(threads), 0, stream, a);
+            } else if (v == 2) {
+                hipLaunchKernelGGL((conv1d_silu_prompt_kernel<2, 4>), grid, dim3(threads), 0, stream, a);
+            } else {
+                hipLaunchKernelGGL((conv1d_silu_prompt_kernel<1, 4>), grid, dim3(threads), 0, stream, a);
+            }
+            check_launch("conv1d_silu_prompt_kernel");
+            return;
+        }
+    }
     hipLaunchKernelGGL(conv1d_silu_kernel, dim3((a.C + threads - 1) / threads), dim3(threads), 0, stream, a);
     check_launch("conv1d_silu_kernel");
 }

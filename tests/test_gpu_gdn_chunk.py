@@ -1,9 +1,12 @@
-"""Prompts through the gated delta rule: the chunked form (more than 16 tokens at head dimension 128) at the
-edges of its 32-token chunks, against the FP64 oracle."""
+"""Prompts through the recurrent-state ops: the chunked gated delta rule (more than 16 tokens at head
+dimension 128) at the edges of its 32-token chunks, and the tiled convolution, against the FP64 oracle."""
 import numpy as np
 import pytest
 
-from test_gpu_gdn import GDN_OUTPUT_BF16, _f, _inputs, _ok, run_regular
+import ninfer_amd as na
+from ninfer_amd import ops
+from ninfer_amd.device import DeviceArray, synchronize
+from test_gpu_gdn import BF16_REDUCTION, GDN_OUTPUT_BF16, _bf, _dev, _f, _inputs, _ok, run_regular
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +60,26 @@ def test_non_finite_token_leaves_earlier_outputs(gpu, where):
     out = _f(run_regular(inp, 128, H, H, T, True, False)[0]).reshape(T, H, 128)
     _ok(out[:40], clean[:40], GDN_OUTPUT_BF16, "out before") # the chunk's products in another order
     assert np.isnan(out[40]).any()
+
+
+@pytest.mark.parametrize("C,T,offset,in_place", [(10240, 17, 0, False), (10240, 1700, 0, True), (1001, 33, 0, True), (64, 16, 0, False),
+                                                 (130, 100, 0, False), (512, 40, 1, True), (24, 19, 0, True)])
+def test_conv_prompt(gpu, C, T, offset, in_place):
+    """Tiles of 16 and 4 tokens, 8, 2 and 1 channels per thread (odd C; tensors one element off), and the
+    window read before it is replaced."""
+    print(f"case conv prompt C={C} T={T} offset={offset} in_place={in_place}", flush=True)
+    from oracle import pyoracle
+    rng = np.random.default_rng(C + T)
+    x, w, win = (_bf(rng.uniform(-2, 2, n)) for n in (T * C, 4 * C, 3 * C))
+
+    def dev(a, shape):
+        d = DeviceArray.from_numpy(na.BF16, np.concatenate([np.zeros(offset, np.uint16), a]))
+        return d, na.Tensor.make(d.ptr + 2 * offset, na.BF16, shape)
+    keep, (tx, tw, tin, to, tout) = zip(*(dev(a, s) for a, s in ((x, (C, T)), (w, (C, 4)), (win, (C, 3)), (win * 0, (C, 3)), (x * 0, (C, T)))))
+    ops.causal_conv1d_silu(tx, tw, tin, tin if in_place else to, tout)
+    synchronize()
+    ref = pyoracle.causal_conv1d_silu(x, w, win, C, T)
+    ref_out = ref[0] if isinstance(ref, tuple) else ref
+    _ok(_f(keep[4].numpy()[offset:]).reshape(T, C), np.asarray(ref_out).reshape(T, C), BF16_REDUCTION, "out")
+    got = keep[2 if in_place else 3].numpy()[offset:].reshape(3, C)
+    assert np.array_equal(got, x.reshape(T, C)[-3:] if T >= 3 else got)
