@@ -51,6 +51,13 @@ inline constexpr int32_t kAttnMaxTokens = 32;
 // us with non-temporal partials against 13.52-13.54 us cached.
 inline constexpr int32_t kAttnCachedPartialKeys = 1024;
 
+// Batch-1 envelopes of up to this many keys (one split of the plan) are one launch: the workgroup that holds a
+// KV head's whole window writes the output, with no partials and no merge. Measured on MI355X (40/8/128,
+// eager calls): 101 keys, T = 1, 10.3 -> 7.1 us; 254 keys, T = 4, 13.4 -> 10.7 us; 24/4/256 BF16, 254 keys
+// 19.9 -> 17.4 us. At two splits and more one workgroup per head is too slow: 521 keys 12.9 against 15.2 us
+// (BF16), 764 keys 13.5 against 15.2 us.
+inline constexpr uint32_t kAttnDirectKeys = kAttnMinKeysPerSplit;
+
 // wide_rows: the INT8 head_dim-128 cache may serve 33..80 query rows (T x G) in one row chunk of
 // five 16-row tiles (one workgroup per CU) instead of several 32-row chunks that each stream every key.
 SplitPlan plan_attention(int32_t Hq, int32_t Hkv, int32_t D, int32_t T, int32_t B,

@@ -133,6 +133,8 @@ struct AttnArgs {
     int32_t split_budget; // B > 1: most splits the batch's keys are cut into per (row chunk, KV head)
     int32_t max_keys; // envelope max_visible_keys (<= max_context <= P): clamps device positions
     float scale_log2; // softmax scale * log2(e)
+    void* out;        // unsplit windows (DIRECT kernels): the rows' outputs, BF16 or FP32
+    int32_t out_f32;
 };
 
 // Keys per split of a batch-1 plan chosen on the device from the actual window, over the `launched`
@@ -915,13 +917,77 @@ __device__ __forceinline__ void write_partial(const State& s, char* smem, int R,
     }
 }
 
+// Rows [r0, r0 + R) of KV head h (row = token * G + head of the group; r0 = t0 * G) straight to the
+// output, for a window that one workgroup holds: the combine of write_partial without the FP16 store.
+// Returns whether a value came out non-finite.
+template <int NT, int D, typename State>
+__device__ __forceinline__ bool write_direct(const State& s, char* smem, int R, int wave, int c, int g, const AttnArgs& a,
+                                             int h, int t0) {
+    constexpr int kRowStride = D + 4;
+    float* sm_o = reinterpret_cast<float*>(smem);  // [kWaves][32][kRowStride]
+    float* sm_m = sm_o + kWaves * 32 * kRowStride; // [32][kWaves]
+    float* sm_l = sm_m + kWaves * 32;              // [32][kWaves]
+    constexpr int UPR = D / 4;
+    constexpr int RPP = 256 / UPR;
+    static_assert(NT <= 2, "one batch of 32 rows");
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int r = 16 * nt + c;
+        if (g == 0) {
+            sm_m[r * kWaves + wave] = s.m[nt] == -INFINITY ? -INFINITY : s.m[nt] * s.rowmul[nt];
+            sm_l[r * kWaves + wave] = s.l[nt][0];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float* dst = sm_o + (wave * 32 + r) * kRowStride + (D / 16) * (4 * g + e);
+#pragma unroll
+            for (int q4 = 0; q4 < D / 64; ++q4) {
+                *reinterpret_cast<f4*>(dst + 4 * q4) =
+                    f4{s.O[nt][4 * q4][e], s.O[nt][4 * q4 + 1][e], s.O[nt][4 * q4 + 2][e], s.O[nt][4 * q4 + 3][e]};
+            }
+        }
+    }
+    __syncthreads();
+    const int d4 = 4 * (static_cast<int>(threadIdx.x) & (UPR - 1));
+    bool bad = false;
+    for (int r = static_cast<int>(threadIdx.x) / UPR; r < R; r += RPP) {
+        const f4 mv = *reinterpret_cast<const f4*>(sm_m + r * kWaves);
+        const f4 lv = *reinterpret_cast<const f4*>(sm_l + r * kWaves);
+        const float M = fmaxf(fmaxf(mv[0], mv[1]), fmaxf(mv[2], mv[3]));
+        f4 o = {0.f, 0.f, 0.f, 0.f};
+        float lsum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const float wgt = mv[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv[w] - M);
+            o += wgt * *reinterpret_cast<const f4*>(sm_o + (w * 32 + r) * kRowStride + d4);
+            lsum = fmaf(lv[w], wgt, lsum);
+        }
+        o = lsum > 0.0f ? o * (1.0f / lsum) : f4{0.f, 0.f, 0.f, 0.f};
+        bad |= !(__builtin_isfinite(lsum) && __builtin_isfinite(o[0]) && __builtin_isfinite(o[1]) && __builtin_isfinite(o[2]) && __builtin_isfinite(o[3]));
+        const int t = t0 + r / a.G;
+        const int64_t oi = static_cast<int64_t>(D) * (h * a.G + r % a.G + static_cast<int64_t>(a.Hq) * t) + d4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (a.out_f32) {
+                static_cast<float*>(a.out)[oi + e] = o[e];
+            } else {
+                static_cast<uint16_t*>(a.out)[oi + e] = f32_to_bf16_bits(o[e]);
+            }
+        }
+    }
+    return bad;
+}
+
 // D = 128: 78 KB of LDS and at most 256 registers, two workgroups per CU. D = 256: 152 KB of LDS,
 // one workgroup (one wave per SIMD) per CU, which leaves 512 registers per lane for the doubled
 // accumulators and chunk registers. NT = 5 (D = 128): 80 query rows (a 16-node tree at group 5)
 // in one workgroup, so every key is streamed once; one wave per SIMD, the Q tile in LDS of its own.
 // One partial of the INT8 kernel: the keys [k0, kend) of sequence b (k0 a multiple of 128) for KV
 // head h and this workgroup's row chunk, into partial slot `slot`.
-template <int NT, int D, bool ONCE, bool CACHED, bool DEV = false>
+template <int D>
+__device__ void direct_rows_exact(const AttnArgs& a, int h, int t0, int R, float* xs);
+
+template <int NT, int D, bool ONCE, bool CACHED, bool DEV = false, bool DIRECT = false>
 __device__ __forceinline__ void partial_segment(const AttnArgs& a, char* smem, int b, int k0, int kend, int slot, int h) {
     constexpr int G = D / 64; // quant groups per row
     using GE = Geo<D>;
@@ -1111,7 +1177,7 @@ __device__ __forceinline__ void partial_segment(const AttnArgs& a, char* smem, i
     float* out_ml = a.part_ml + pidx * (2 * RMAX);
 
 
-    if (k0 >= hend && !owner) {
+    if (!DIRECT && k0 >= hend && !owner) {
         __builtin_amdgcn_s_waitcnt(0);
         if (threadIdx.x < RMAX) {
             out_ml[2 * threadIdx.x] = -INFINITY;
@@ -1254,7 +1320,13 @@ __device__ __forceinline__ void partial_segment(const AttnArgs& a, char* smem, i
     __builtin_amdgcn_s_waitcnt(0); // no DMA may land in the ring after this point
     __syncthreads();
     static_assert(kWaves * 32 * (D + 4 + 2) * 4 <= GE::kSmemBytes, "wave merge exceeds the LDS map");
-    write_partial<NT, D, CACHED>(s, smem, R, wave, c, g, out_o, out_ml, *kwide_word != 0);
+    if constexpr (DIRECT) {
+        const bool wide = *kwide_word != 0; // a K scale of 512 or more
+        const bool bad = write_direct<NT, D>(s, smem, R, wave, c, g, a, h, t0);
+        if (__syncthreads_or(bad || wide)) { direct_rows_exact<D>(a, h, t0, R, reinterpret_cast<float*>(smem)); }
+    } else {
+        write_partial<NT, D, CACHED>(s, smem, R, wave, c, g, out_o, out_ml, *kwide_word != 0);
+    }
 }
 
 // CACHED: the batch-1 partials go out with ordinary (cached) stores; an instance of its own, launched
@@ -1303,6 +1375,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 &&
     }
 }
 
+// A batch-1 window of up to kAttnDirectKeys keys: one workgroup per (KV head, row chunk) walks all of it and
+// writes the output itself, so the call is one launch. Grid (KV head, 1, row chunk).
+template <int NT, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 1, D == 128 ? 2 : 1))) void verify_attn_direct_kernel(AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[Geo<D>::kSmemBytes];
+    partial_segment<NT, D, false, false, false, true>(a, smem, 0, 0, a.kps, 0, blockIdx.x);
+}
 
 // ---- BF16 KV cache -------------------------------------------------------------------------------
 //
@@ -1517,7 +1596,8 @@ __device__ __forceinline__ void pv_chunk_b(const float (&p)[NT][8], const ChunkR
     }
 }
 
-template <int NT, int D, bool ONCE>
+// DIRECT: one workgroup holds the whole window and writes the output (as verify_attn_direct_kernel).
+template <int NT, int D, bool ONCE, bool DIRECT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void verify_attn_partial_bf16_kernel(AttnArgs a) {
     using GB = GeoB<D>;
     __shared__ __attribute__((aligned(16))) char smem[GB::kSmemBytes];
@@ -1621,7 +1701,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int64_t pidx = (static_cast<int64_t>(rc) * a.Hkv + h) * a.split_slots + slot0 + split;
     uint16_t* out_o = a.part_o + pidx * (32 * D);
     float* out_ml = a.part_ml + pidx * 64;
-    if (k0 >= hend && !owner) {
+    if (!DIRECT && k0 >= hend && !owner) {
         __builtin_amdgcn_s_waitcnt(0);
         if (threadIdx.x < 32) {
             out_ml[2 * threadIdx.x] = -INFINITY;
@@ -1734,7 +1814,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     static_assert(kWaves * 32 * (D + 4 + 2) * 4 <= GB::kSmemBytes, "wave merge exceeds the LDS map");
-    write_partial<NT, D, false>(s, smem, R, wave, c, g, out_o, out_ml);
+    if constexpr (DIRECT) {
+        (void)write_direct<NT, D>(s, smem, R, wave, c, g, a, h, t0);
+    } else {
+        write_partial<NT, D, false>(s, smem, R, wave, c, g, out_o, out_ml);
+    }
 }
 
 struct MergeArgs {
@@ -1886,6 +1970,47 @@ __device__ void exact_split(const MergeArgs& a, int b, int t, int qh, int k0, in
     m_out = M;
     l_out = Ls;
     o_out = Od;
+}
+
+// The rows of an unsplit window that its FP16 operands could not hold, again and exactly: rows
+// [t0 * G, t0 * G + R) of KV head h.
+template <int D>
+__device__ void direct_rows_exact(const AttnArgs& a, int h, int t0, int R, float* xs) {
+    MergeArgs m{};
+    m.T = a.T;
+    m.Hq = a.Hq;
+    m.Hkv = a.Hkv;
+    m.G = a.G;
+    m.q = a.q;
+    m.positions = a.positions;
+    m.parents = a.parents;
+    m.kc = a.kc;
+    m.vc = a.vc;
+    m.ks = a.ks;
+    m.vs = a.vs;
+    m.P = a.P;
+    m.max_keys = a.max_keys;
+    m.fused = a.k_new != nullptr ? 1 : 0;
+    m.scale_log2 = a.scale_log2;
+    __syncthreads(); // the appended rows and the first outputs are written
+#pragma unroll 1
+    for (int i = 0; i < R * (D / 32); ++i) {
+        const int r = i / (D / 32);
+        const int d0 = 32 * (i % (D / 32));
+        const int t = t0 + r / a.G;
+        const int qh = h * a.G + r % a.G;
+        float M, L, O;
+        exact_split<D>(m, 0, t, qh, 0, a.kps, d0, xs, M, L, O);
+        if (threadIdx.x < 32) {
+            const float val = L > 0.0f ? O / L : 0.0f;
+            const int64_t oi = static_cast<int64_t>(D) * (qh + static_cast<int64_t>(a.Hq) * t) + d0 + threadIdx.x;
+            if (a.out_f32) {
+                static_cast<float*>(a.out)[oi] = val;
+            } else {
+                static_cast<uint16_t*>(a.out)[oi] = f32_to_bf16_bits(val);
+            }
+        }
+    }
 }
 
 // The merge of one output row's 32-dim slice over its splits in split order (running log-sum-exp),
@@ -2493,6 +2618,38 @@ void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uin
     // One row chunk: every key is read by exactly one workgroup (non-temporal DMAs).
     const bool once = plan.row_chunks == 1;
     const int rows = plan.tokens_per_chunk * plan.G;
+    a.out = out;
+    a.out_f32 = out_f32 ? 1 : 0;
+    if (c.B == 1 && plan.rows_per_slot == kAttnRowsPerTile && max_keys <= kAttnDirectKeys) {
+        a.kps = static_cast<int32_t>((max_keys + 127) / 128 * 128);
+        const dim3 one(c.Hkv, 1, plan.row_chunks);
+        const bool small = rows <= 16;
+        if (c.kb != nullptr && c.D == 128) {
+            if (small) {
+                hipLaunchKernelGGL((verify_attn_partial_bf16_kernel<1, 128, false, true>), one, dim3(256), 0, stream, a);
+            } else {
+                hipLaunchKernelGGL((verify_attn_partial_bf16_kernel<2, 128, false, true>), one, dim3(256), 0, stream, a);
+            }
+        } else if (c.kb != nullptr) {
+            if (small) {
+                hipLaunchKernelGGL((verify_attn_partial_bf16_kernel<1, 256, false, true>), one, dim3(256), 0, stream, a);
+            } else {
+                hipLaunchKernelGGL((verify_attn_partial_bf16_kernel<2, 256, false, true>), one, dim3(256), 0, stream, a);
+            }
+        } else if (c.D == 128) {
+            if (small) {
+                hipLaunchKernelGGL((verify_attn_direct_kernel<1, 128>), one, dim3(256), 0, stream, a);
+            } else {
+                hipLaunchKernelGGL((verify_attn_direct_kernel<2, 128>), one, dim3(256), 0, stream, a);
+            }
+        } else if (small) {
+            hipLaunchKernelGGL((verify_attn_direct_kernel<1, 256>), one, dim3(256), 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((verify_attn_direct_kernel<2, 256>), one, dim3(256), 0, stream, a);
+        }
+        check_launch("verify_attn_direct_kernel");
+        return;
+    }
     const dim3 grid_split_major(plan.split_slots, c.Hkv, plan.row_chunks);
     // the batch-1 paths (BF16, and INT8 of up to two row tiles) take (KV head, split, row chunk)
     const dim3 grid_b1(c.Hkv, plan.split_slots, plan.row_chunks);
