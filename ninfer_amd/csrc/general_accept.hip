@@ -27,6 +27,8 @@
 //   4 gen_nucleus  per column: crossing value, rank cut, kstar and nucleus mass
 //   5 gen_totals   per draw tile: accept decision (recomputed per block), masses of the draw
 //   6 gen_pick     per sequence: locate the draw, commit the round
+// Batches with enough columns replace 1-4 by one launch: gen_column finds a whole column's nucleus in one
+// workgroup (see there).
 #include "common.h"
 #include "device_utils.h"
 #include "general_internal.h"
@@ -92,7 +94,7 @@ struct GenArgs {
     struct DraftEntry* dtab;
 };
 
-// Inputs of draft i's accept test, gathered once per round by gen_coarse so that no later launch
+// Inputs of draft i's accept test, gathered once per round by gen_coarse or gen_column so that no later launch
 // waits on drafts -> logits: the BF16 bits of target column i and draft column i at token d_i
 // (xpq = xp | xq << 16, zero outside the token domain) and d_i itself (-1 outside the domain).
 struct DraftEntry {
@@ -424,6 +426,428 @@ __global__ __launch_bounds__(kThreads) void gen_nucleus_kernel(GenArgs a) {
     }
 }
 
+// ---- 1-4 in one launch: a workgroup per column ---------------------------------------------------
+// The weight depends on a token's BF16 value only, so a column needs one exponential per distinct value (a few
+// thousand) and not per token: the values are counted in LDS, one atomic per token; maximum, total mass,
+// crossing value and rank cut follow from the counts without leaving the workgroup, and one more walk over
+// the column finds the id of the last included token. Word r of the histogram counts magnitude r, positive
+// in its low half and negative in its high half: the raw bits are the address, and what bounds both walks is the
+// vector instructions per token on one CU. So it pays once there are columns for a good part of the
+// chip; with few the tile launches spread each column over every CU. MI355X, 112 columns (K = 3, batch 16,
+// V = 248,320): one launch of 44 us where max, coarse, fine and nucleus took 75; the call 100 -> 75 us. Of the 44,
+// counting takes 16, the group masses 9, the id walk 11, clearing and the sample 3.
+// A magnitude with more than 65,535 tokens of one sign overflows its counter: the counts then sum below V (a
+// wrap loses 65,535 or 65,536), and the column is counted again in 512 groups with a weight per token.
+constexpr int kColThreads = 1024;
+constexpr int kColWaves = kColThreads / 64;
+constexpr int kGroups = 512;     // groups of 128 consecutive values in ordered16's order
+constexpr int kSegment = 512;    // tokens of a segment in the search for the last included one
+constexpr uint32_t kOrderedInf = 0xff80u, kOrderedNegInf = 0x007fu; // ordered16 of the infinities
+constexpr uint32_t kNoCommon = 0x10000u; // no token's bits
+constexpr int kAhead = 8;        // 16-byte loads in flight per thread in a walk
+constexpr int kBatch = 8 * kColThreads * kAhead;
+constexpr int kMaxBatches = (kGenTile * kGenMaxTiles + kBatch - 1) / kBatch;
+
+using u16x2 = unsigned short __attribute__((ext_vector_type(2)));
+using s16x2 = short __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t ordered_of_bits(uint32_t raw) {
+    return raw == 0x8000u ? 0x8000u : ((raw & 0x8000u) ? (~raw & 0xffffu) : (raw | 0x8000u)); // -0 counts as +0
+}
+
+// A column in batches of kBatch tokens, first to last or last to first, until done(batch number) holds after a
+// batch (asked of every thread alike): f8(words, v0) for the 8 tokens from v0 in a 16-byte aligned column,
+// read kAhead loads at once without a branch around them; f1(bits, v) for its last V % 8 tokens and for
+// every token of a column at another address.
+template <bool BACKWARD, typename F8, typename F1, typename Done>
+__device__ __forceinline__ void walk_column(const uint16_t* col, int V, F8&& f8, F1&& f1, Done&& done) {
+    const int tid = static_cast<int>(threadIdx.x);
+    const bool aligned = (reinterpret_cast<uintptr_t>(col) & 15u) == 0;
+    const int full = aligned ? V & ~7 : 0;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(col), 0, 2 * full, 0x00020000);
+    const int batches = (V + kBatch - 1) / kBatch;
+    for (int n = 0; n < batches; ++n) {
+        const int base = kBatch * (BACKWARD ? batches - 1 - n : n);
+        if (aligned) {
+            i4 w[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                w[k] = __builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(
+                    rsrc, 2 * (base + 8 * (k * kColThreads + tid)), 0, 0));
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int v0 = base + 8 * (k * kColThreads + tid);
+                if (v0 < full) { f8(w[k], v0); }
+            }
+        }
+        const int last = min(base + kBatch, V);
+        for (int v = max(base, full) + tid; v < last; v += kColThreads) { f1(static_cast<uint32_t>(col[v]), v); }
+        if (done(n)) { break; }
+    }
+}
+
+// Maximum over the workgroup, in every thread.
+__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* red) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) { v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, 64))); }
+    if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = v; }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kColWaves; ++w) { v = max(v, red[w]); }
+    return v;
+}
+
+// Every token, one at a time: for the rare columns (NaN, a wrapped counter), kept small beside the hot walks.
+template <typename F1>
+__device__ __forceinline__ void walk_tokens(const uint16_t* col, int V, F1&& f1) {
+#pragma unroll 1
+    for (int v = static_cast<int>(threadIdx.x); v < V; v += kColThreads) { f1(static_cast<uint32_t>(col[v])); }
+}
+
+__global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
+    __shared__ __attribute__((aligned(16))) uint32_t hist[32768];
+    __shared__ uint64_t gmass[kGroups];
+    __shared__ uint32_t gcount[kGroups];
+    __shared__ uint32_t fine[128];
+    __shared__ uint32_t scount[kGenTile * kGenMaxTiles / kSegment];
+    __shared__ uint32_t found[kMaxBatches];
+    __shared__ uint64_t wsum[kColWaves];
+    __shared__ uint32_t wmax[kColWaves];
+    __shared__ int first;
+    __shared__ uint32_t common_bits, common_count;
+    __shared__ uint64_t bcast[4];
+    const int c = blockIdx.x, b = blockIdx.y;
+    const int64_t cb = static_cast<int64_t>(b) * a.ncols + c;
+    const int tid = static_cast<int>(threadIdx.x);
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const uint16_t* col = column_ptr(a, b, c);
+    if (c == 0 && tid < a.K) {
+        const int d = a.drafts[b * a.K + tid];
+        const bool in_domain = d >= 0 && d < a.V;
+        const uint32_t xp = in_domain ? column_ptr(a, b, tid)[d] : 0u;
+        const uint32_t xq = in_domain ? column_ptr(a, b, a.K + 1 + tid)[d] : 0u;
+        a.dtab[static_cast<int64_t>(b) * a.K + tid] = DraftEntry{xp | (xq << 16), in_domain ? d : -1};
+    }
+    for (int i = tid; i < 32768 / 4; i += kColThreads) { reinterpret_cast<i4*>(hist)[i] = i4{0, 0, 0, 0}; }
+    if (tid == 0) {
+        first = kGroups;
+        common_bits = kNoCommon;
+        common_count = 0u;
+    }
+    __syncthreads();
+    // A value that many tokens share (a mask's) would serialize its LDS atomics: if 1,024 tokens across the column
+    // hold one 64 times, its tokens are counted in registers. The sample's own counts are taken back. 112 columns
+    // with 50% of the tokens masked: 86 us against 108 for the tile passes. Columns of a few distinct values keep
+    // conflicts (logits rounded to integers: 196 against 104 us).
+    {
+        const uint32_t raw = col[static_cast<int64_t>(tid) * a.V / kColThreads];
+        const uint32_t one = 1u + 65535u * (raw >> 15);
+        const uint32_t old = atomicAdd(&hist[raw & 0x7fffu], one);
+        if (((raw >> 15) ? old >> 16 : old & 0xffffu) >= 63u) { atomicMin(&common_bits, raw); }
+        __syncthreads();
+        atomicSub(&hist[raw & 0x7fffu], one);
+        __syncthreads();
+    }
+    const uint32_t common = common_bits;
+    // The maximum is the greatest signed pattern if that is not negative, else the least unsigned one.
+    s16x2 hi = {-32768, -32768};
+    u16x2 lo = {65535, 65535};
+    if (common == kNoCommon) {
+        walk_column<false>(
+            col, a.V,
+            [&](const i4& w, int) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t p = static_cast<uint32_t>(w[i]);
+                    hi = __builtin_elementwise_max(hi, __builtin_bit_cast(s16x2, p));
+                    lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u16x2, p));
+                    atomicAdd(&hist[p & 0x7fffu], 1u + 65535u * ((p >> 15) & 1u));
+                    atomicAdd(&hist[(p >> 16) & 0x7fffu], 1u + 65535u * (p >> 31));
+                }
+            },
+            [&](uint32_t raw, int) {
+                hi.x = max(hi.x, static_cast<short>(raw));
+                lo.x = min(lo.x, static_cast<unsigned short>(raw));
+                atomicAdd(&hist[raw & 0x7fffu], 1u + 65535u * (raw >> 15));
+            },
+            [](int) { return false; });
+    } else {
+        uint32_t mine = 0;
+        const auto count_token = [&](uint32_t raw, int) {
+            hi.x = max(hi.x, static_cast<short>(raw));
+            lo.x = min(lo.x, static_cast<unsigned short>(raw));
+            if (raw == common) {
+                ++mine;
+            } else {
+                atomicAdd(&hist[raw & 0x7fffu], 1u + 65535u * (raw >> 15));
+            }
+        };
+        walk_column<false>(
+            col, a.V,
+            [&](const i4& w, int v0) {
+#pragma unroll 1
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t p = static_cast<uint32_t>(i < 2 ? (i == 0 ? w[0] : w[1]) : (i == 2 ? w[2] : w[3]));
+                    count_token(p & 0xffffu, v0);
+                    count_token(p >> 16, v0);
+                }
+            },
+            count_token, [](int) { return false; });
+        mine = wave_inclusive_scan(mine);
+        if (lane == 63) { atomicAdd(&common_count, mine); }
+    }
+    const short top = max(hi.x, hi.y);
+    uint32_t omax = ordered_of_bits(top >= 0 ? static_cast<uint32_t>(top) : static_cast<uint32_t>(min(lo.x, lo.y)));
+    omax = block_max_u32(omax, wmax);
+    if (omax > kOrderedInf || omax < kOrderedNegInf) { // NaN among the tokens: the maximum is taken without them
+        omax = kOrderedNegInf;
+        walk_tokens(col, a.V, [&](uint32_t raw) {
+            if ((raw & 0x7fffu) <= 0x7f80u) { omax = max(omax, ordered_of_bits(raw)); }
+        });
+        __syncthreads();
+        omax = block_max_u32(omax, wmax);
+    }
+    ColDesc d{};
+    d.inv_temp = 1.0f / a.config->temperature;
+    d.m = value_of_ordered16(omax) * d.inv_temp;
+    const float top_p = a.config->top_p;
+
+    // ---- group counts and masses: a wave reads the magnitudes of two exponents at once, 32 lanes to each, 4
+    // words to a lane; most of the range is empty
+    uint32_t seen = 0;
+    for (int e2 = wave; e2 < kGroups / 4; e2 += kColWaves) {
+        const i4 w = reinterpret_cast<const i4*>(hist)[64 * e2 + lane];
+        uint64_t mass[2] = {0, 0};
+        uint32_t n[2] = {0, 0};
+        if (__any((w[0] | w[1] | w[2] | w[3]) != 0)) {
+            const uint32_t mag = 4u * (64u * e2 + lane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t pos = static_cast<uint32_t>(w[i]) & 0xffffu;
+                uint32_t neg = static_cast<uint32_t>(w[i]) >> 16;
+                if (mag + i == 0u) {
+                    pos += neg;
+                    neg = 0;
+                }
+                n[0] += pos;
+                n[1] += neg;
+                if (pos != 0u) { mass[0] += pos * gen_weight(value_of_ordered16(0x8000u + mag + i), d.inv_temp, d.m); }
+                if (neg != 0u) { mass[1] += neg * gen_weight(value_of_ordered16(0x7fffu - mag - i), d.inv_temp, d.m); }
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int off = 1; off < 32; off <<= 1) {
+                    mass[s] += __shfl_xor(static_cast<unsigned long long>(mass[s]), off, 64);
+                    n[s] += static_cast<uint32_t>(__shfl_xor(static_cast<int>(n[s]), off, 64));
+                }
+            }
+        }
+        if ((lane & 31) == 0) {
+            const int e = 2 * e2 + (lane >> 5);
+            gmass[256 + e] = mass[0];
+            gcount[256 + e] = n[0];
+            gmass[255 - e] = mass[1];
+            gcount[255 - e] = n[1];
+            seen += n[0] + n[1];
+        }
+    }
+    seen += static_cast<uint32_t>(__shfl_xor(static_cast<int>(seen), 32, 64));
+    if (lane == 0) { wsum[wave] = seen; }
+    __syncthreads();
+    uint64_t counted = 0;
+#pragma unroll
+    for (int w = 0; w < kColWaves; ++w) { counted += wsum[w]; }
+    const uint32_t shared = common_count;
+    const bool exact = counted + shared == static_cast<uint64_t>(a.V);
+    if (!exact) { // a counter wrapped
+        __syncthreads();
+        for (int i = tid; i < kGroups; i += kColThreads) {
+            gmass[i] = 0;
+            gcount[i] = 0;
+        }
+        __syncthreads();
+        walk_tokens(col, a.V, [&](uint32_t raw) {
+            if (raw == common) { return; }
+            const uint32_t o = ordered_of_bits(raw);
+            atomicAdd(&gcount[o >> 7], 1u);
+            atomicAdd(reinterpret_cast<unsigned long long*>(&gmass[o >> 7]),
+                      static_cast<unsigned long long>(gen_weight(value_of_ordered16(o), d.inv_temp, d.m)));
+        });
+        __syncthreads();
+    }
+
+    const uint32_t common_o = shared != 0u ? ordered_of_bits(common) : 0u;
+    if (shared != 0u && tid == kGroups - 1 - static_cast<int>(common_o >> 7)) { // its group's owner below
+        gcount[common_o >> 7] += shared;
+        gmass[common_o >> 7] += shared * gen_weight(value_of_ordered16(common_o), d.inv_temp, d.m);
+    }
+
+    // ---- total mass; the group (descending values) in which the running mass reaches the target
+    const int gi = kGroups - 1 - tid; // threads < 512 own one group each
+    const uint64_t mass = tid < kGroups ? gmass[gi] : 0ull;
+    const uint32_t count = tid < kGroups ? gcount[gi] : 0u;
+    uint64_t incl = wave_inclusive_scan(mass);
+    __syncthreads(); // wsum's earlier use is over
+    if (lane == 63) { wsum[wave] = incl; }
+    __syncthreads();
+    uint64_t Z = 0;
+#pragma unroll
+    for (int w = 0; w < kColWaves; ++w) {
+        if (w < wave) { incl += wsum[w]; }
+        Z += wsum[w];
+    }
+    d.z = Z;
+    d.zs = Z;
+    if (!(top_p < 1.0f)) {
+        if (tid == 0) {
+            d.c1 = -1;
+            a.desc[cb] = d;
+        }
+        return;
+    }
+    const uint64_t target = static_cast<uint64_t>((static_cast<u128>(Z) * fixed_u24(top_p)) >> 24);
+    if (count != 0u && incl >= target) { atomicMin(&first, tid); }
+    __syncthreads();
+    const int f = first;
+    if (f >= kGroups) { // no finite mass
+        if (tid == 0) { a.desc[cb] = d; }
+        return;
+    }
+    const int group = kGroups - 1 - f;
+    if (tid == f) { bcast[0] = incl - mass; }
+    if (!exact) {
+        if (tid < 128) { fine[tid] = 0u; }
+        __syncthreads();
+        walk_tokens(col, a.V, [&](uint32_t raw) {
+            const uint32_t o = ordered_of_bits(raw);
+            if (raw != common && static_cast<int>(o >> 7) == group) { atomicAdd(&fine[o & 127u], 1u); }
+        });
+    } else if (tid < 128) {
+        if (group >= 256) {
+            const uint32_t w = hist[128 * (group - 256) + tid];
+            fine[tid] = (w & 0xffffu) + (group == 256 && tid == 0 ? w >> 16 : 0u);
+        } else {
+            const int mag = 0x7fff - 128 * group - tid;
+            fine[tid] = mag != 0 ? hist[mag] >> 16 : 0u;
+        }
+    }
+    __syncthreads();
+
+    if (shared != 0u && tid == 0 && static_cast<int>(common_o >> 7) == group) { fine[common_o & 127u] += shared; }
+    __syncthreads();
+
+    // ---- crossing value inside the group (wave 0: lane l owns values 127 - 2l and 126 - 2l) and the rank cut
+    if (wave == 0) {
+        const uint64_t above = bcast[0];
+        uint64_t n[2], wt[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t v = 127u - 2u * lane - k;
+            n[k] = fine[v];
+            wt[k] = n[k] != 0ull ? gen_weight(value_of_ordered16(128u * group + v), d.inv_temp, d.m) : 0ull;
+        }
+        const uint64_t both = n[0] * wt[0] + n[1] * wt[1];
+        const uint64_t before0 = above + wave_inclusive_scan(both) - both;
+        const uint64_t before1 = before0 + n[0] * wt[0];
+        const bool hit0 = n[0] != 0ull && before1 >= target;
+        const bool hit1 = n[1] != 0ull && before1 + n[1] * wt[1] >= target;
+        const unsigned long long m = __ballot(hit0 || hit1);
+        if (m != 0ull && lane == __ffsll(static_cast<long long>(m)) - 1) {
+            const int k = hit0 ? 0 : 1;
+            const uint64_t before = hit0 ? before0 : before1;
+            // smallest j >= 1 with before + j * w >= target (w > 0 at the crossing)
+            uint64_t j = target > before ? (target - before + wt[k] - 1) / wt[k] : 0;
+            j = j < 1 ? 1 : (j > n[k] ? n[k] : j);
+            bcast[1] = n[k] - j;
+            bcast[2] = before + j * wt[k];
+            bcast[3] = 128u * group + 127u - 2u * lane - k;
+        }
+    }
+    __syncthreads();
+    const uint32_t vstar = static_cast<uint32_t>(bcast[3]);
+
+    // ---- the j-th token of value vstar (ids ascending) = the one with `after` more behind it. Last batch first:
+    // it is the one that L2 still holds, and the walk ends at the batch that has it.
+    const uint32_t after = static_cast<uint32_t>(bcast[1]);
+    const int segments = (a.V + kSegment - 1) / kSegment;
+    for (int i = tid; i < segments; i += kColThreads) { scount[i] = 0u; }
+    if (tid < kMaxBatches) { found[tid] = 0u; }
+    __syncthreads();
+    // Bits of the value and what to leave out of the compare: the sign of zero.
+    const uint32_t bits = vstar >= 0x8000u ? vstar - 0x8000u : 0xffffu - vstar;
+    const uint32_t keep = bits == 0u ? 0x7fffu : 0xffffu;
+    const uint32_t bits2 = bits | (bits << 16), keep2 = keep | (keep << 16);
+    uint32_t mine = 0, behind = 0;
+    walk_column<true>(
+        col, a.V,
+        [&](const i4& w, int v0) {
+            uint32_t x[4];
+            u16x2 any = {65535, 65535}; // zero in a half: a match
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[i] = (static_cast<uint32_t>(w[i]) & keep2) ^ bits2;
+                any = __builtin_elementwise_min(any, __builtin_bit_cast(u16x2, x[i]));
+            }
+            if (any.x == 0 || any.y == 0) {
+                uint32_t n = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { n += ((x[i] & 0xffffu) == 0u) + ((x[i] >> 16) == 0u); }
+                atomicAdd(&scount[v0 / kSegment], n);
+                mine += n;
+            }
+        },
+        [&](uint32_t raw, int v) {
+            if ((raw & keep) == bits) {
+                atomicAdd(&scount[v / kSegment], 1u);
+                ++mine;
+            }
+        },
+        [&](int n) { // a batch has a counter of its own: nobody writes what others still read
+            if (mine != 0u) { atomicAdd(&found[n], mine); }
+            mine = 0;
+            __syncthreads();
+            behind += found[n];
+            return behind > after;
+        });
+    if (wave != 0) { return; }
+    uint32_t run = 0;
+    int seg = -1;
+    for (int s0 = 0; s0 < segments; s0 += 64) {
+        const int at = segments - 1 - s0 - lane;
+        const uint32_t n = at >= 0 ? scount[at] : 0u;
+        const uint32_t in = run + wave_inclusive_scan(n);
+        const unsigned long long m = __ballot(in > after);
+        if (m != 0ull) {
+            const int src = __ffsll(static_cast<long long>(m)) - 1;
+            seg = segments - 1 - s0 - src;
+            run = static_cast<uint32_t>(__shfl(static_cast<int>(in - n), src, 64));
+            break;
+        }
+        run = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(in), 63));
+    }
+    if (seg < 0) { return; }
+    const int v0 = kSegment * seg + 8 * lane;
+    uint32_t hits = 0; // bit e: token v0 + e has the value
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if (v0 + e < a.V && (col[v0 + e] & keep) == bits) { hits |= 1u << e; }
+    }
+    const uint32_t n = static_cast<uint32_t>(__popc(hits));
+    const uint32_t in = wave_inclusive_scan(n);
+    const uint32_t all = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(in), 63));
+    const uint32_t rank = all - (after - run); // 1-based within the segment
+    if (n != 0u && in >= rank && in - n < rank) {
+        for (uint32_t need = rank - (in - n); need > 1; --need) { hits &= hits - 1; }
+        d.kstar = sort_key(value_of_ordered16(vstar), v0 + __ffs(static_cast<int>(hits)) - 1);
+        d.zs = bcast[2];
+        d.nucleus = 1;
+        a.desc[cb] = d;
+    }
+}
+
 // Accept decisions of sequence b (identical in every block that evaluates them), from the
 // sequence's descriptors in LDS (sd) and thread i's draft entry e and accept uniform ua: thread
 // i < K tests draft i, and the first failing draft is the rejection. Returns a; sets *rejected to the
@@ -735,14 +1159,19 @@ void launch_general_accept(const GenLaunch& l, const GenPlan& plan, void* worksp
     a.dtab = reinterpret_cast<DraftEntry*>(ws + plan.dtab_offset);
     const dim3 tiles(plan.ntiles, plan.ncols, l.B);
     const dim3 cols(plan.ncols, l.B);
-    hipLaunchKernelGGL(gen_max_kernel, tiles, dim3(kThreads), 0, stream, a);
-    check_launch("gen_max_kernel");
-    hipLaunchKernelGGL(gen_coarse_kernel, tiles, dim3(kThreads), 0, stream, a);
-    check_launch("gen_coarse_kernel");
-    hipLaunchKernelGGL(gen_fine_kernel, tiles, dim3(kThreads), 0, stream, a);
-    check_launch("gen_fine_kernel");
-    hipLaunchKernelGGL(gen_nucleus_kernel, cols, dim3(kThreads), 0, stream, a);
-    check_launch("gen_nucleus_kernel");
+    if (plan.ncols * l.B >= kGenColumnMin) {
+        hipLaunchKernelGGL(gen_column_kernel, cols, dim3(kColThreads), 0, stream, a);
+        check_launch("gen_column_kernel");
+    } else {
+        hipLaunchKernelGGL(gen_max_kernel, tiles, dim3(kThreads), 0, stream, a);
+        check_launch("gen_max_kernel");
+        hipLaunchKernelGGL(gen_coarse_kernel, tiles, dim3(kThreads), 0, stream, a);
+        check_launch("gen_coarse_kernel");
+        hipLaunchKernelGGL(gen_fine_kernel, tiles, dim3(kThreads), 0, stream, a);
+        check_launch("gen_fine_kernel");
+        hipLaunchKernelGGL(gen_nucleus_kernel, cols, dim3(kThreads), 0, stream, a);
+        check_launch("gen_nucleus_kernel");
+    }
     hipLaunchKernelGGL(gen_totals_kernel, dim3(plan.ndraw, l.B), dim3(kThreads), 0, stream, a);
     check_launch("gen_totals_kernel");
     hipLaunchKernelGGL(gen_pick_kernel, dim3(l.B), dim3(kThreads), 0, stream, a);
