@@ -160,7 +160,8 @@ size_t nmi_gqa_attention_workspace_bytes(int32_t q_heads, int32_t kv_heads, int3
  * (include/ninfer/ops/gqa_attention.h:50; src/ops/wrapper/gqa_attention.cpp:229-245), as a status
  * plus the size: the geometry follows from q_heads (24 -> 4 KV heads and 16 -> 2 at head_dim 256,
  * the reference's registered ones; 40 -> 8 at head_dim 128), and the size covers every execution
- * envelope of one sequence (above 32 tokens: the prompt route's launches of 32 and its last one).
+ * envelope of one sequence (above 32 tokens: what the prompt route's launches of 32 and its last one take;
+ * the prompt kernel's key splits use as much of that as they need).
  * tokens <= 0 give 0; other q_heads NMI_INVALID_ARGUMENT. */
 int nmi_gqa_attention_workspace_bound(int32_t q_heads, int32_t tokens, size_t* bytes);
 
@@ -169,7 +170,8 @@ int nmi_gqa_attention_workspace_bound(int32_t q_heads, int32_t tokens, size_t* b
  * q/out BF16 [D, Hq, T(, B)]; k/v BF16 [D, Hkv, T(, B)]; positions I32 [T(, B)] sequential;
  * out may also be FP32 (EXTENSION). T above 32 is the reference's prompt route
  * (src/ops/wrapper/gqa_attention.cpp:202-213): one sequence (B = 1); the rows are appended first,
- * then the tokens attend in launches of 32 through the same workspace. */
+ * then the tokens attend through the same workspace: in one prompt kernel (and a merge where it splits the
+ * keys), or in verify launches of 32 for short prompts and for q, out or cache planes off 16 bytes. */
 int nmi_gqa_attention(const nmi_tensor* q, const nmi_tensor* k, const nmi_tensor* v,
                       const nmi_tensor* positions, float scale, const nmi_kv_layer_view* cache,
                       nmi_gqa_envelope envelope, void* workspace, size_t workspace_bytes,
