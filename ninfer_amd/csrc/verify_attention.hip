@@ -102,6 +102,8 @@ __device__ __forceinline__ float partial_o_at(const uint16_t* base, int64_t i) {
     return partial_o_half(partial_o_word(base, i), i);
 }
 
+constexpr int kXcds = 8; // each with an L2 of its own
+
 struct AttnArgs {
     const uint16_t* q;
     const uint16_t* k_new; // fused A1 append (single row chunk only): BF16 [D, Hkv, T, B]
@@ -135,6 +137,7 @@ struct AttnArgs {
     float scale_log2; // softmax scale * log2(e)
     void* out;        // unsplit windows (DIRECT kernels): the rows' outputs, BF16 or FP32
     int32_t out_f32;
+    int32_t interleaved; // B == 1, BF16 cache of head_dim 256: one-dimensional grid of interleaved_part
 };
 
 // Keys per split of a batch-1 plan chosen on the device from the actual window, over the `launched`
@@ -1596,6 +1599,24 @@ __device__ __forceinline__ void pv_chunk_b(const float (&p)[NT][8], const ChunkR
     }
 }
 
+// Several row chunks at batch 1: each (KV head, split) has a workgroup per row chunk, all streaming the same keys,
+// and workgroups go to the 8 XCDs in turn. Where KV heads x splits is a multiple of 8 the grid (KV head, split, row
+// chunk) puts those workgroups on one XCD, whose L2 serves all but the first; elsewhere they are numbered 8
+// apart in a one-dimensional grid. MI355X, 24/4/256 over 32,774 keys, T = 6 (29 splits): 51.6 -> 40.6 us;
+// 190,000 keys 150 -> 148 us.
+// The INT8 kernel is not bound by these reads and was 4 to 13% slower numbered so. Returns whether the
+// workgroup has a part.
+__device__ __forceinline__ bool interleaved_part(const AttnArgs& a, int& h, int& split, int& rc) {
+    const uint32_t place = blockIdx.x / kXcds;
+    const uint32_t group = place / static_cast<uint32_t>(a.row_chunks);
+    const uint32_t unit = group * kXcds + blockIdx.x % kXcds;
+    const uint32_t heads = static_cast<uint32_t>(a.Hkv);
+    split = static_cast<int>(unit / heads);
+    h = static_cast<int>(unit % heads);
+    rc = static_cast<int>(place - group * static_cast<uint32_t>(a.row_chunks));
+    return split < a.split_slots;
+}
+
 // DIRECT: one workgroup holds the whole window and writes the output (as verify_attn_direct_kernel).
 template <int NT, int D, bool ONCE, bool DIRECT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void verify_attn_partial_bf16_kernel(AttnArgs a) {
@@ -1607,10 +1628,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int c = lane & 15;
     const int g = lane >> 4;
     // B = 1: grid (KV head, split, row chunk), as in the INT8 kernel; batches: (slot, KV head, row chunk)
-    const int h = a.B == 1 ? blockIdx.x : blockIdx.y;
-    const int rc = blockIdx.z;
+    int h = a.B == 1 ? blockIdx.x : blockIdx.y;
+    int rc = blockIdx.z;
     int b = 0;
     int split = a.B == 1 ? blockIdx.y : blockIdx.x;
+    if constexpr (D == 256 && !ONCE && !DIRECT) {
+        if (a.interleaved != 0 && !interleaved_part(a, h, split, rc)) { return; }
+    }
     int kps = a.kps;
     int slot0 = 0;
     if (a.B > 1) {
@@ -2676,6 +2700,13 @@ void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uin
     const bool dev = plan.b1_device_plan;
     if (c.kb != nullptr) {
         if (c.B == 1) { grid = grid_b1; }
+        // Short windows read too little to gain (704 keys 19.3 against 19.5 us, 2,106 keys 19.9 against 19.7), and
+        // head_dim 128 runs two workgroups per CU (T = 16 over 21,500 keys: 53.6 against 54.5 us).
+        const int units = c.Hkv * plan.split_slots;
+        if (c.B == 1 && c.D == 256 && !once && max_keys > 2048 && units % kXcds != 0) {
+            a.interleaved = 1;
+            grid = dim3((units + kXcds - 1) / kXcds * kXcds * plan.row_chunks);
+        }
         if (c.D == 128) {
             if (rows <= 16) {
                 NMI_PARTIAL(verify_attn_partial_bf16_kernel, 1, 128)
