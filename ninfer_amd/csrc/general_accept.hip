@@ -433,17 +433,28 @@ __global__ __launch_bounds__(kThreads) void gen_nucleus_kernel(GenArgs a) {
 // the column finds the id of the last included token. Word r of the histogram counts magnitude r, positive
 // in its low half and negative in its high half: the raw bits are the address, and what bounds both walks is the
 // vector instructions per token on one CU. So it pays once there are columns for a good part of the
-// chip; with few the tile launches spread each column over every CU. MI355X, 112 columns (K = 3, batch 16,
-// V = 248,320): one launch of 44 us where max, coarse, fine and nucleus took 75; the call 100 -> 75 us. Of the 44,
-// counting takes 16, the group masses 9, the id walk 11, clearing and the sample 3.
+// chip; with few the tile launches spread each column over every CU. Whole call on MI355X, K = 3, V = 248,320,
+// tile launches -> this one: 70 columns 72.5 -> 61.6 us, 112 97.5 -> 67.6, 224 158 -> 82.
 // A magnitude with more than 65,535 tokens of one sign overflows its counter: the counts then sum below V (a
 // wrap loses 65,535 or 65,536), and the column is counted again in 512 groups with a weight per token.
+// Values that many tokens share (a mask's, logits on a grid) would serialize their LDS atomics: logits rounded to
+// integers took 191 us at 112 columns, and 547 with half of the tokens masked. So a sample of 1,024 tokens finds up
+// to kHot of them, and if there are enough, every token looks its value up in a tag table indexed by a hash of the
+// bits (lanes that read one word do not conflict) and counts a frequent one in a word per (value, lane). 112 columns,
+// tile launches -> now: integers 99.6 -> 75.3 us, half masked 104 -> 77, both 103 -> 76, steps of 1/8 98 -> 77,
+// of 1/16 98 -> 79, of 1/32 97 -> 83, two values 125 -> 63. (70 columns in steps of 1/32 72.5 -> 78: nearly as many
+// values as kHot holds, and conflicts left.)
 constexpr int kColThreads = 1024;
 constexpr int kColWaves = kColThreads / 64;
 constexpr int kGroups = 512;     // groups of 128 consecutive values in ordered16's order
 constexpr int kSegment = 512;    // tokens of a segment in the search for the last included one
 constexpr uint32_t kOrderedInf = 0xff80u, kOrderedNegInf = 0x007fu; // ordered16 of the infinities
-constexpr uint32_t kNoCommon = 0x10000u; // no token's bits
+constexpr int kHot = 128;        // most frequent values counted apart
+constexpr int kHotLanes = 32;    // counters of one (lane l and l + 32 share one)
+constexpr uint32_t kHotAt = 8;   // of 1,024 sampled tokens: a value counts as frequent
+constexpr uint32_t kHotOne = 80; // one value this frequent, or kHotFew frequent ones: they are counted apart
+constexpr uint32_t kHotFew = 24;
+constexpr int kTags = 1024;
 constexpr int kAhead = 8;        // 16-byte loads in flight per thread in a walk
 constexpr int kBatch = 8 * kColThreads * kAhead;
 constexpr int kMaxBatches = (kGenTile * kGenMaxTiles + kBatch - 1) / kBatch;
@@ -456,7 +467,7 @@ __device__ __forceinline__ uint32_t ordered_of_bits(uint32_t raw) {
 }
 
 // A column in batches of kBatch tokens, first to last or last to first, until done(batch number) holds after a
-// batch (asked of every thread alike): f8(words, v0) for the 8 tokens from v0 in a 16-byte aligned column,
+// batch (asked of every thread alike): f8(words, v0, load) for the 8 tokens from v0 in a 16-byte aligned column,
 // read kAhead loads at once without a branch around them; f1(bits, v) for its last V % 8 tokens and for
 // every token of a column at another address.
 template <bool BACKWARD, typename F8, typename F1, typename Done>
@@ -478,7 +489,7 @@ __device__ __forceinline__ void walk_column(const uint16_t* col, int V, F8&& f8,
 #pragma unroll
             for (int k = 0; k < kAhead; ++k) {
                 const int v0 = base + 8 * (k * kColThreads + tid);
-                if (v0 < full) { f8(w[k], v0); }
+                if (v0 < full) { f8(w[k], v0, k); }
             }
         }
         const int last = min(base + kBatch, V);
@@ -498,6 +509,11 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* red) {
     return v;
 }
 
+// Bucket of a value in the tag table, and the 24-bit hash multipliers to choose from (0 hashes to bucket 0 and 2
+// does not, under each).
+__device__ __forceinline__ uint32_t tag_bucket(uint32_t raw, uint32_t mul) { return __umul24(raw, mul) >> 14 & (kTags - 1); }
+__device__ __forceinline__ uint32_t tag_multiplier(int i) { return 10368889u + 246914u * static_cast<uint32_t>(i); }
+
 // Every token, one at a time: for the rare columns (NaN, a wrapped counter), kept small beside the hot walks.
 template <typename F1>
 __device__ __forceinline__ void walk_tokens(const uint16_t* col, int V, F1&& f1) {
@@ -506,16 +522,23 @@ __device__ __forceinline__ void walk_tokens(const uint16_t* col, int V, F1&& f1)
 }
 
 __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
-    __shared__ __attribute__((aligned(16))) uint32_t hist[32768];
+    constexpr int kHotWords = kHot * kHotLanes;
+    constexpr int kHotAt0 = kTags, kHistAt = kTags + kHotWords;
+    __shared__ __attribute__((aligned(16))) uint32_t words[kHistAt + 32768];
+    uint32_t* const tags = words; // per bucket: a frequent value's bits | index of its counters << 16
+    uint32_t* const hot = words + kHotAt0; // [kHot][kHotLanes], packed as the histogram's words
+    uint32_t* const hist = words + kHistAt;
+    uint32_t* const scount = hot; // segment counts, once the counters are summed
+    static_assert(kGenTile * kGenMaxTiles / kSegment <= kHotWords, "segment counts");
     __shared__ uint64_t gmass[kGroups];
     __shared__ uint32_t gcount[kGroups];
     __shared__ uint32_t fine[128];
-    __shared__ uint32_t scount[kGenTile * kGenMaxTiles / kSegment];
     __shared__ uint32_t found[kMaxBatches];
     __shared__ uint64_t wsum[kColWaves];
     __shared__ uint32_t wmax[kColWaves];
+    __shared__ uint32_t hot_bits[kHot], hot_count[kHot];
     __shared__ int first;
-    __shared__ uint32_t common_bits, common_count;
+    __shared__ uint32_t hot_n, hot_top, hot_hash;
     __shared__ uint64_t bcast[4];
     const int c = blockIdx.x, b = blockIdx.y;
     const int64_t cb = static_cast<int64_t>(b) * a.ncols + c;
@@ -530,34 +553,75 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         const uint32_t xq = in_domain ? column_ptr(a, b, a.K + 1 + tid)[d] : 0u;
         a.dtab[static_cast<int64_t>(b) * a.K + tid] = DraftEntry{xp | (xq << 16), in_domain ? d : -1};
     }
-    for (int i = tid; i < 32768 / 4; i += kColThreads) { reinterpret_cast<i4*>(hist)[i] = i4{0, 0, 0, 0}; }
+    for (int i = tid; i < (kHistAt + 32768) / 4; i += kColThreads) { reinterpret_cast<i4*>(words)[i] = i4{0, 0, 0, 0}; }
+    uint32_t* taken = gcount; // [kColWaves][kTags / 32] bits: the group counts are not in use yet
+    static_assert(kColWaves * kTags / 32 == kGroups, "bucket bits");
+    if (tid < kGroups) { taken[tid] = 0u; }
     if (tid == 0) {
         first = kGroups;
-        common_bits = kNoCommon;
-        common_count = 0u;
+        hot_n = 0u;
+        hot_top = 0u;
+        hot_hash = 0xffffffffu;
     }
     __syncthreads();
-    // A value that many tokens share (a mask's) would serialize its LDS atomics: if 1,024 tokens across the column
-    // hold one 64 times, its tokens are counted in registers. The sample's own counts are taken back. 112 columns
-    // with 50% of the tokens masked: 86 us against 108 for the tile passes. Columns of a few distinct values keep
-    // conflicts (logits rounded to integers: 196 against 104 us).
+    // The sample's own counts are taken back.
+    const uint32_t sample = col[static_cast<int64_t>(tid) * a.V / kColThreads];
+    const uint32_t sample_one = 1u + 65535u * (sample >> 15);
     {
-        const uint32_t raw = col[static_cast<int64_t>(tid) * a.V / kColThreads];
-        const uint32_t one = 1u + 65535u * (raw >> 15);
-        const uint32_t old = atomicAdd(&hist[raw & 0x7fffu], one);
-        if (((raw >> 15) ? old >> 16 : old & 0xffffu) >= 63u) { atomicMin(&common_bits, raw); }
-        __syncthreads();
-        atomicSub(&hist[raw & 0x7fffu], one);
+        const uint32_t old = atomicAdd(&hist[sample & 0x7fffu], sample_one);
+        const uint32_t seen = (sample >> 15) ? old >> 16 : old & 0xffffu;
+        if (seen == kHotAt - 1) {
+            const uint32_t slot = atomicAdd(&hot_n, 1u);
+            if (slot < kHot) { hot_bits[slot] = sample; }
+        }
+        if (seen == kHotOne - 1) { hot_top = 1u; }
         __syncthreads();
     }
-    const uint32_t common = common_bits;
+    const bool few = hot_top != 0u || hot_n >= kHotFew;
+    const int nhot = few ? static_cast<int>(min(hot_n, static_cast<uint32_t>(kHot))) : 0;
+    uint32_t mul = 0;
+    if (few) {
+        // A wave per multiplier: the tokens whose bucket is taken already. The best one fills the table, the more
+        // frequent value first; one that loses its bucket keeps its histogram word, and its counters stay empty.
+        const auto sampled = [&](uint32_t raw) {
+            const uint32_t n = hist[raw & 0x7fffu];
+            return (raw >> 15) ? n >> 16 : n & 0xffffu;
+        };
+        uint32_t lost = 0;
+        for (int i = lane; i < nhot; i += 64) {
+            const uint32_t b0 = tag_bucket(hot_bits[i], tag_multiplier(wave));
+            const uint32_t old = atomicOr(&taken[kTags / 32 * wave + (b0 >> 5)], 1u << (b0 & 31u));
+            if ((old >> (b0 & 31u)) & 1u) { lost += sampled(hot_bits[i]); }
+        }
+        lost = wave_inclusive_scan(lost);
+        if (lane == 63) { atomicMin(&hot_hash, (lost << 4) | static_cast<uint32_t>(wave)); }
+        __syncthreads();
+        mul = tag_multiplier(static_cast<int>(hot_hash & 15u));
+        if (tid < nhot) {
+            const uint32_t raw = hot_bits[tid];
+            atomicMax(&tags[tag_bucket(raw, mul)], (min(sampled(raw), 511u) << 23) | (static_cast<uint32_t>(tid) << 16) | raw);
+        }
+        __syncthreads();
+        // The slot becomes the index of its counters; an empty bucket holds bits that hash elsewhere.
+        static_assert(kTags == kColThreads, "a bucket per thread");
+        const uint32_t t = tags[tid];
+        tags[tid] = t >> 23 != 0u ? (kHotAt0 + ((t >> 16) & (kHot - 1)) * kHotLanes) << 16 | (t & 0xffffu) : (tid == 0 ? 2u : 0u);
+    }
+    atomicSub(&hist[sample & 0x7fffu], sample_one);
+    __syncthreads();
+    static_assert(kColWaves == 16 && kHot == 128, "tag and multiplier fields");
+    // Values on a grid leave the low mantissa bits zero, so where there are frequent values the exponent's low bits
+    // pick the word within its group as well, and with it the LDS bank.
+    const uint32_t swz = few ? 7u : 0u;
+    const auto word_of = [&](uint32_t mag) { return mag ^ ((mag >> 7) & swz); };
+    const auto is_hot = [&](uint32_t raw) { return few && (tags[tag_bucket(raw, mul)] & 0xffffu) == raw; };
     // The maximum is the greatest signed pattern if that is not negative, else the least unsigned one.
     s16x2 hi = {-32768, -32768};
     u16x2 lo = {65535, 65535};
-    if (common == kNoCommon) {
+    if (!few) {
         walk_column<false>(
             col, a.V,
-            [&](const i4& w, int) {
+            [&](const i4& w, int, int) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const uint32_t p = static_cast<uint32_t>(w[i]);
@@ -574,29 +638,36 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
             },
             [](int) { return false; });
     } else {
-        uint32_t mine = 0;
-        const auto count_token = [&](uint32_t raw, int) {
-            hi.x = max(hi.x, static_cast<short>(raw));
-            lo.x = min(lo.x, static_cast<unsigned short>(raw));
-            if (raw == common) {
-                ++mine;
-            } else {
-                atomicAdd(&hist[raw & 0x7fffu], 1u + 65535u * (raw >> 15));
-            }
+        const uint32_t hot_lane = lane & (kHotLanes - 1);
+        const auto count_token = [&](uint32_t raw, uint32_t tag) {
+            const bool h = (tag & 0xffffu) == raw;
+            const uint32_t in_hot = (tag >> 16) + hot_lane, in_hist = ((raw & 0x7fffu) ^ ((raw >> 7) & 7u)) + kHistAt;
+            const uint32_t at = __builtin_unpredictable(h) ? in_hot : in_hist;
+            atomicAdd(&words[at], 1u + 65535u * (raw >> 15));
         };
         walk_column<false>(
             col, a.V,
-            [&](const i4& w, int v0) {
-#pragma unroll 1
+            [&](const i4& w, int, int) {
+                uint32_t raw[8], tag[8];
+#pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t p = static_cast<uint32_t>(i < 2 ? (i == 0 ? w[0] : w[1]) : (i == 2 ? w[2] : w[3]));
-                    count_token(p & 0xffffu, v0);
-                    count_token(p >> 16, v0);
+                    const uint32_t p = static_cast<uint32_t>(w[i]);
+                    hi = __builtin_elementwise_max(hi, __builtin_bit_cast(s16x2, p));
+                    lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u16x2, p));
+                    raw[2 * i] = p & 0xffffu;
+                    raw[2 * i + 1] = p >> 16;
                 }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { tag[i] = tags[tag_bucket(raw[i], mul)]; }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { count_token(raw[i], tag[i]); }
             },
-            count_token, [](int) { return false; });
-        mine = wave_inclusive_scan(mine);
-        if (lane == 63) { atomicAdd(&common_count, mine); }
+            [&](uint32_t raw, int) {
+                hi.x = max(hi.x, static_cast<short>(raw));
+                lo.x = min(lo.x, static_cast<unsigned short>(raw));
+                count_token(raw, tags[tag_bucket(raw, mul)]);
+            },
+            [](int) { return false; });
     }
     const short top = max(hi.x, hi.y);
     uint32_t omax = ordered_of_bits(top >= 0 ? static_cast<uint32_t>(top) : static_cast<uint32_t>(min(lo.x, lo.y)));
@@ -622,19 +693,20 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         uint64_t mass[2] = {0, 0};
         uint32_t n[2] = {0, 0};
         if (__any((w[0] | w[1] | w[2] | w[3]) != 0)) {
-            const uint32_t mag = 4u * (64u * e2 + lane);
+            const uint32_t word = 4u * (64u * e2 + lane);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
+                const uint32_t mag = word_of(word + i);
                 uint32_t pos = static_cast<uint32_t>(w[i]) & 0xffffu;
                 uint32_t neg = static_cast<uint32_t>(w[i]) >> 16;
-                if (mag + i == 0u) {
+                if (mag == 0u) {
                     pos += neg;
                     neg = 0;
                 }
                 n[0] += pos;
                 n[1] += neg;
-                if (pos != 0u) { mass[0] += pos * gen_weight(value_of_ordered16(0x8000u + mag + i), d.inv_temp, d.m); }
-                if (neg != 0u) { mass[1] += neg * gen_weight(value_of_ordered16(0x7fffu - mag - i), d.inv_temp, d.m); }
+                if (pos != 0u) { mass[0] += pos * gen_weight(value_of_ordered16(0x8000u + mag), d.inv_temp, d.m); }
+                if (neg != 0u) { mass[1] += neg * gen_weight(value_of_ordered16(0x7fffu - mag), d.inv_temp, d.m); }
             }
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
@@ -655,13 +727,22 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         }
     }
     seen += static_cast<uint32_t>(__shfl_xor(static_cast<int>(seen), 32, 64));
+    // the frequent values' counts, two to a wave
+    for (int i = 2 * wave; i < nhot; i += 2 * kColWaves) {
+        const uint32_t w = hot[kHotLanes * i + lane]; // one value's: one half is zero
+        const uint32_t n = wave_inclusive_scan((w & 0xffffu) + (w >> 16));
+        const uint32_t n0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(n), 31));
+        const uint32_t n1 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(n), 63));
+        if (lane == 0) { hot_count[i] = n0; }
+        if (lane == 1) { hot_count[i + 1] = n1 - n0; }
+        seen += n1;
+    }
     if (lane == 0) { wsum[wave] = seen; }
     __syncthreads();
     uint64_t counted = 0;
 #pragma unroll
     for (int w = 0; w < kColWaves; ++w) { counted += wsum[w]; }
-    const uint32_t shared = common_count;
-    const bool exact = counted + shared == static_cast<uint64_t>(a.V);
+    const bool exact = counted == static_cast<uint64_t>(a.V);
     if (!exact) { // a counter wrapped
         __syncthreads();
         for (int i = tid; i < kGroups; i += kColThreads) {
@@ -670,7 +751,7 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         }
         __syncthreads();
         walk_tokens(col, a.V, [&](uint32_t raw) {
-            if (raw == common) { return; }
+            if (is_hot(raw)) { return; }
             const uint32_t o = ordered_of_bits(raw);
             atomicAdd(&gcount[o >> 7], 1u);
             atomicAdd(reinterpret_cast<unsigned long long*>(&gmass[o >> 7]),
@@ -679,11 +760,17 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         __syncthreads();
     }
 
-    const uint32_t common_o = shared != 0u ? ordered_of_bits(common) : 0u;
-    if (shared != 0u && tid == kGroups - 1 - static_cast<int>(common_o >> 7)) { // its group's owner below
-        gcount[common_o >> 7] += shared;
-        gmass[common_o >> 7] += shared * gen_weight(value_of_ordered16(common_o), d.inv_temp, d.m);
+    uint32_t my_hot = 0u, my_o = 0u; // thread i: frequent value i
+    if (tid < nhot) {
+        my_hot = hot_count[tid];
+        my_o = ordered_of_bits(hot_bits[tid]);
+        if (my_hot != 0u) {
+            atomicAdd(&gcount[my_o >> 7], my_hot);
+            atomicAdd(reinterpret_cast<unsigned long long*>(&gmass[my_o >> 7]),
+                      static_cast<unsigned long long>(my_hot * gen_weight(value_of_ordered16(my_o), d.inv_temp, d.m)));
+        }
     }
+    __syncthreads();
 
     // ---- total mass; the group (descending values) in which the running mass reaches the target
     const int gi = kGroups - 1 - tid; // threads < 512 own one group each
@@ -723,20 +810,20 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
         __syncthreads();
         walk_tokens(col, a.V, [&](uint32_t raw) {
             const uint32_t o = ordered_of_bits(raw);
-            if (raw != common && static_cast<int>(o >> 7) == group) { atomicAdd(&fine[o & 127u], 1u); }
+            if (static_cast<int>(o >> 7) == group && !is_hot(raw)) { atomicAdd(&fine[o & 127u], 1u); }
         });
     } else if (tid < 128) {
         if (group >= 256) {
-            const uint32_t w = hist[128 * (group - 256) + tid];
+            const uint32_t w = hist[word_of(128u * (group - 256) + tid)];
             fine[tid] = (w & 0xffffu) + (group == 256 && tid == 0 ? w >> 16 : 0u);
         } else {
             const int mag = 0x7fff - 128 * group - tid;
-            fine[tid] = mag != 0 ? hist[mag] >> 16 : 0u;
+            fine[tid] = mag != 0 ? hist[word_of(mag)] >> 16 : 0u;
         }
     }
     __syncthreads();
 
-    if (shared != 0u && tid == 0 && static_cast<int>(common_o >> 7) == group) { fine[common_o & 127u] += shared; }
+    if (my_hot != 0u && static_cast<int>(my_o >> 7) == group) { atomicAdd(&fine[my_o & 127u], my_hot); }
     __syncthreads();
 
     // ---- crossing value inside the group (wave 0: lane l owns values 127 - 2l and 126 - 2l) and the rank cut
@@ -780,34 +867,42 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
     const uint32_t bits = vstar >= 0x8000u ? vstar - 0x8000u : 0xffffu - vstar;
     const uint32_t keep = bits == 0u ? 0x7fffu : 0xffffu;
     const uint32_t bits2 = bits | (bits << 16), keep2 = keep | (keep << 16);
-    uint32_t mine = 0, behind = 0;
+    // Load k of a batch gives wave w the whole segment 16k + w: a lane's matches of two segments share a word, and the
+    // wave sums them once per batch.
+    static_assert(kSegment == 8 * 64 && kAhead % 2 == 0, "a wave's load is a segment");
+    uint32_t pair[kAhead / 2] = {}, lone = 0, behind = 0;
     walk_column<true>(
         col, a.V,
-        [&](const i4& w, int v0) {
-            uint32_t x[4];
-            u16x2 any = {65535, 65535}; // zero in a half: a match
+        [&](const i4& w, int, int k) {
+            u16x2 miss = {0, 0};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                x[i] = (static_cast<uint32_t>(w[i]) & keep2) ^ bits2;
-                any = __builtin_elementwise_min(any, __builtin_bit_cast(u16x2, x[i]));
+                const uint32_t x = (static_cast<uint32_t>(w[i]) & keep2) ^ bits2;
+                miss += __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), u16x2{1, 1});
             }
-            if (any.x == 0 || any.y == 0) {
-                uint32_t n = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) { n += ((x[i] & 0xffffu) == 0u) + ((x[i] >> 16) == 0u); }
-                atomicAdd(&scount[v0 / kSegment], n);
-                mine += n;
-            }
+            pair[k / 2] += (8u - miss.x - miss.y) << (16 * (k & 1));
         },
         [&](uint32_t raw, int v) {
-            if ((raw & keep) == bits) {
-                atomicAdd(&scount[v / kSegment], 1u);
-                ++mine;
-            }
+            // the wave's tokens here are 64 consecutive ones of a segment, or fewer than 8
+            const uint32_t n = static_cast<uint32_t>(__popcll(__ballot((raw & keep) == bits)));
+            if (lane == 0 && n != 0u) { atomicAdd(&scount[v / kSegment], n); }
+            lone += n;
         },
         [&](int n) { // a batch has a counter of its own: nobody writes what others still read
-            if (mine != 0u) { atomicAdd(&found[n], mine); }
-            mine = 0;
+            const int s0 = kBatch / kSegment * (static_cast<int>((a.V + kBatch - 1) / kBatch) - 1 - n) + wave;
+            uint32_t all = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lone)));
+#pragma unroll
+            for (int j = 0; j < kAhead / 2; ++j) {
+                const uint32_t sum = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(wave_inclusive_scan(pair[j])), 63));
+                if (lane == 0 && sum != 0u) {
+                    if ((sum & 0xffffu) != 0u) { atomicAdd(&scount[s0 + kColWaves * 2 * j], sum & 0xffffu); }
+                    if (sum >> 16 != 0u) { atomicAdd(&scount[s0 + kColWaves * (2 * j + 1)], sum >> 16); }
+                }
+                all += (sum & 0xffffu) + (sum >> 16);
+                pair[j] = 0;
+            }
+            lone = 0;
+            if (lane == 0 && all != 0u) { atomicAdd(&found[n], all); }
             __syncthreads();
             behind += found[n];
             return behind > after;

@@ -13,8 +13,8 @@ inline constexpr int32_t kGenDescBytes = 64;    // per-column nucleus descriptor
 inline constexpr int32_t kGenDraftEntryBytes = 8; // per-draft accept-test inputs
 // Columns of a batch from which one workgroup per column replaces the tile passes. The tile passes grow with the
 // columns, a workgroup per column takes about the same time until there is more than one for every CU. Whole
-// call, V = 248,320, tiles / columns: 28 columns 50 / 59 us, 56: 66 / 67 us, 70: 76 / 68 us, 112: 101 / 75 us,
-// 240: 166 / 88 us. At V = 4,096 both take about 40 us.
+// call, V = 248,320, tiles / columns: 28 columns 50 / 59 us, 56: 66 / 67, 70: 73 / 62, 112: 98 / 68, 224: 158 / 82;
+// V = 32,000: 70 columns 35 / 31, 224 46 / 33; V = 1,000 to 4,096: 34 to 37 / 28 at any of these.
 inline constexpr int32_t kGenColumnMin = 64;
 
 // Workspace layout, shared by the size query and the launch.

@@ -5,8 +5,23 @@ import numpy as np
 
 import ninfer_amd as na
 from ninfer_amd import ops
-from ninfer_amd.device import DeviceArray, DeviceBuffer, Stream
+from ninfer_amd.device import DeviceArray, DeviceBuffer, Event, Stream, synchronize
 from ninfer_amd.kv_cache import KVCacheLayer
+
+
+def time_us(call, reps=20, rounds=5) -> float:
+    """Device time of one call: the best of `rounds` event-timed runs of `reps` calls (stream, default)."""
+    call()
+    best = float("inf")
+    for _ in range(rounds):
+        a, b = Event(), Event()
+        a.record(None)
+        for _ in range(reps):
+            call()
+        b.record(None)
+        synchronize()
+        best = min(best, a.elapsed_ms(b) * 1e3 / reps)
+    return best
 
 
 def upload_cache(case) -> KVCacheLayer:
@@ -114,8 +129,9 @@ def run_accept(logits, drafts, length, stats, token_domain, cfgs, target_tokens=
     return out
 
 
-def run_general(target, draft, drafts, u_accept, u_residual, length, stats, token_domain, temperature, top_p):
-    """Mode F batch acceptance. target uint16 [B][K+1][rows]; draft uint16 [B][K][rows]."""
+def run_general(target, draft, drafts, u_accept, u_residual, length, stats, token_domain, temperature, top_p, timed=False):
+    """Mode F batch acceptance. target uint16 [B][K+1][rows]; draft uint16 [B][K][rows]. `timed`: the call's
+    device time in us instead of its outputs."""
     target = np.asarray(target, dtype=np.uint16)
     draft = np.asarray(draft, dtype=np.uint16)
     B, Kp1, rows = target.shape
@@ -139,10 +155,14 @@ def run_general(target, draft, drafts, u_accept, u_residual, length, stats, toke
     cfg_buf.upload(np.frombuffer(bytes(memoryview(cfg)), dtype=np.uint8))
     ws = DeviceBuffer(ops.general_accept_workspace_bytes(token_domain, K, B))
     ws.fill(0xFF)  # the op may not depend on what scratch held before
-    ops.speculative_accept_general(d_t.tensor(), d_d.tensor(), d_dr.tensor(), d_ua.tensor(), d_ur.tensor(),
-                                   d_len.tensor(), d_tok.tensor(), d_so.tensor(), d_ns.tensor(), d_acc.tensor(),
-                                   d_stats.tensor(), token_domain, cfg_buf.ptr, ws)
-    from ninfer_amd.device import synchronize
+    views = [x.tensor() for x in (d_t, d_d, d_dr, d_ua, d_ur, d_len, d_tok, d_so, d_ns, d_acc, d_stats)]
+
+    def call():
+        ops.speculative_accept_general(*views, token_domain, cfg_buf.ptr, ws)
+
+    if timed:
+        return time_us(call)
+    call()
     synchronize()
     return dict(sampled_out=d_so.numpy().reshape(B, K + 1), num_sampled=d_ns.numpy(), accepted=d_acc.numpy(),
                 token=d_tok.numpy(), length=d_len.numpy(), stats=d_stats.numpy().reshape(B, -1))
