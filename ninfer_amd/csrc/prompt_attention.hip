@@ -45,6 +45,7 @@ namespace nmi {
 namespace {
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+using u16x2 = unsigned short __attribute__((ext_vector_type(2)));
 
 struct PromptArgs {
     const uint16_t* q;
@@ -84,7 +85,8 @@ struct PromptGeo {
     static constexpr int kRowV = 2 * KT;         // LDS bytes of one V^T row
     static constexpr int kPlane = 32768;         // one K or V^T plane of a tile
     static constexpr int kBuf = 2 * kPlane;
-    static constexpr int kSmem = 2 * kBuf + 64;
+    // the flag of a second walk, and its bit per key tile: a cache plane of 2^31 bytes has 131,072 tiles
+    static constexpr int kSmem = 2 * kBuf + 131072 / 8;
     static_assert(NCH % WK == 0, "every wave takes whole chunks");
 };
 
@@ -173,14 +175,13 @@ __device__ __forceinline__ void load_tile(const HeadPlanes<D, BF>& hp, int key0,
 }
 
 // Decode a thread's part into an LDS buffer. Keys at or past `window` get zero V values (those rows
-// may hold anything; their scores are masked). Returns the FP32-range test bits of the live K scales.
+// may hold anything; their scores are masked). `top` collects the largest bits of the live INT8 scales.
 template <int D, bool BF>
-__device__ __forceinline__ uint32_t store_tile(const TileRegs<D, BF>& r, char* buf, int key0, int window, int tid) {
+__device__ __forceinline__ void store_tile(const TileRegs<D, BF>& r, char* buf, int key0, int window, int tid, u16x2& top) {
     using PG = PromptGeo<D, BF, 1>;
     const int dq = tid % (D / 4);
     const int oct = tid / (D / 4);
     const int kv0 = key0 + 32 * (oct >> 2) + 4 * (oct & 3);
-    uint32_t wide = 0u;
     char* vp = buf + PG::kPlane;
     if constexpr (!BF) {
 #pragma unroll
@@ -189,7 +190,7 @@ __device__ __forceinline__ uint32_t store_tile(const TileRegs<D, BF>& r, char* b
             const int key = u / (D / 16);
             const int piece = u % (D / 16);
             const uint32_t sc = r.ksc[i] & 0xffffu;
-            wide |= key0 + key < window ? sc & (sc << 1) : 0u;
+            top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, key0 + key < window ? sc : 0u));
             const h2 s2 = __builtin_bit_cast(h2, sc | (sc << 16));
             char* row = buf + key * PG::kRowK;
             *reinterpret_cast<h8*>(row + 16 * (piece ^ (key & 15))) =
@@ -205,6 +206,8 @@ __device__ __forceinline__ uint32_t store_tile(const TileRegs<D, BF>& r, char* b
                 if (kv0 + (j & 3) + 16 * (j >> 2) >= window) { vsp[j >> 1][j & 1] = static_cast<_Float16>(0.0f); }
             }
         }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) { top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, vsp[w])); }
         const auto put = [&](auto byte) {
             constexpr int B = decltype(byte)::value;
             h2 pr[4];
@@ -243,8 +246,10 @@ __device__ __forceinline__ uint32_t store_tile(const TileRegs<D, BF>& r, char* b
             *reinterpret_cast<u4*>(vp + d * PG::kRowV + 16 * v_slot<D>(oct, d)) = pr;
         }
     }
-    return wide;
 }
+
+// A scale of 512 or more (an FP16 exponent of 24), NaN included.
+__device__ __forceinline__ bool wide_scale(u16x2 top) { return max(top.x, top.y) >= 0x6000; }
 
 // Online-softmax state of one wave.
 template <int D, bool BF, int NT>
@@ -258,92 +263,273 @@ struct PromptRows {
     f4 O[NT][D / 16];  // O^T: tile t entry e of lane (c, g) is dim 16t + 4g + e of row 16nt + c
 };
 
-// The exact form of one row (FP32(code) * scale, FP32 arithmetic; reference decode
-// include/ninfer/ops/gqa_attention.h:30), for tiles the FP16 operands could not hold. Whole workgroup.
-template <int D>
-__device__ void prompt_exact_row(const PromptArgs& a, int h, int t, int qh, int last, float* xs) {
-    constexpr int GQ = D / 64;
-    constexpr int PARTS = kPromptThreads / D;
-    float* xq = xs;
-    float* xp = xs + D;
-    float* xr = xp + kPromptThreads;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int dim = tid % D;
-    const int part = tid / D;
-    const int64_t orow = static_cast<int64_t>(D) * (qh + static_cast<int64_t>(a.Hq) * t);
-    const int8_t* kbase = a.kc + static_cast<int64_t>(h) * a.P * D;
-    const int8_t* vbase = a.vc + static_cast<int64_t>(h) * a.P * D;
-    const uint16_t* ksb = a.ks + static_cast<int64_t>(h) * a.P * GQ;
-    const uint16_t* vsb = a.vs + static_cast<int64_t>(h) * a.P * GQ;
-    __syncthreads();
-    if (tid < D) { xq[tid] = bf16_to_f32(a.q[orow + tid]) * a.scale_log2; }
-    __syncthreads();
-    const int n = last + 1;
-    float M = -INFINITY, L = 0.0f, O = 0.0f;
-    for (int base = 0; base < n; base += kPromptThreads) {
-        const int key = base + tid;
-        float sc = -INFINITY;
-        if (key < n) {
-            sc = 0.0f;
-            for (int gq = 0; gq < GQ; ++gq) {
-                const float ksc = f16_bits_to_f32(ksb[static_cast<int64_t>(key) * GQ + gq]);
-                float p = 0.0f;
-                for (int d = 0; d < 64; ++d) {
-                    p = fmaf(xq[64 * gq + d], static_cast<float>(kbase[static_cast<int64_t>(key) * D + 64 * gq + d]) * ksc, p);
+// S^T = K' Q^T of chunk ci of the tile in `buf`.
+template <int D, bool BF, int NT>
+__device__ __forceinline__ void chunk_scores(const char* buf, int ci, int c, int g, const PromptRows<D, BF, NT>& s, f4 (&sacc)[2][NT]) {
+    using PG = PromptGeo<D, BF, 1>;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+        const char* krow = buf + (32 * ci + 16 * kt + c) * PG::kRowK;
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks) {
+            const u4 ka = *reinterpret_cast<const u4*>(krow + 16 * ((4 * ks + g) ^ c));
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const f4 acc = ks == 0 ? f4{0.f, 0.f, 0.f, 0.f} : sacc[kt][nt];
+                if constexpr (BF) {
+                    sacc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, ka), __builtin_bit_cast(bf8, s.q[nt][ks]), acc, 0, 0, 0);
+                } else {
+                    sacc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, s.q[nt][ks]), acc, 0, 0, 0);
                 }
-                sc += p;
             }
-        }
-        const float wm = wave_max(sc);
-        if (lane == 0) { xr[wave] = wm; }
-        __syncthreads();
-        float Mn = M;
-        for (int w = 0; w < kPromptThreads / 64; ++w) { Mn = fmaxf(Mn, xr[w]); }
-        const float alpha = (M == -INFINITY || Mn == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
-        const float p = (sc == -INFINITY || Mn == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(sc - Mn);
-        xp[tid] = p;
-        const float wsum = wave_sum(p);
-        if (lane == 0) { xr[8 + wave] = wsum; }
-        __syncthreads();
-        float bs = 0.0f;
-        for (int w = 0; w < kPromptThreads / 64; ++w) { bs += xr[8 + w]; }
-        L = fmaf(L, alpha, bs);
-        float acc = 0.0f;
-        for (int j = 0; j < kPromptThreads / PARTS; ++j) {
-            const int i = part * (kPromptThreads / PARTS) + j;
-            const int k = base + i;
-            if (k < n && xp[i] != 0.0f) {
-                acc = fmaf(xp[i], static_cast<float>(vbase[static_cast<int64_t>(k) * D + dim]) *
-                                      f16_bits_to_f32(vsb[static_cast<int64_t>(k) * GQ + dim / 64]), acc);
-            }
-        }
-        O = fmaf(O, alpha, acc);
-        M = Mn;
-        __syncthreads(); // xp and xr are reused
-    }
-    xp[tid] = O;
-    __syncthreads();
-    if (tid < D) {
-        float o = 0.0f;
-        for (int w = 0; w < PARTS; ++w) { o += xp[w * D + tid]; }
-        const float val = L > 0.0f ? o / L : 0.0f;
-        if (a.out_f32) {
-            static_cast<float*>(a.out)[orow + tid] = val;
-        } else {
-            static_cast<uint16_t*>(a.out)[orow + tid] = f32_to_bf16_bits(val);
         }
     }
 }
 
-template <int D, bool BF, int WK>
-__global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prompt_attn_kernel(PromptArgs a) {
+// The chunk's scores (-inf where the key is past the row's last one), and the lazy rescale of the state to its
+// running maximum (constants and rounding as in verify_attention.hip).
+template <int D, bool BF, int NT>
+__device__ __forceinline__ void chunk_rescale(const f4 (&sacc)[2][NT], int c0, bool masked, int g, PromptRows<D, BF, NT>& s, float (&sv)[NT][8]) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { sv[nt][i] = sacc[i >> 2][nt][i & 3]; }
+    }
+    if (masked) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int key = c0 + 16 * (i >> 2) + 4 * g + (i & 3);
+                sv[nt][i] = key <= s.pos[nt] ? sv[nt][i] : -INFINITY;
+            }
+        }
+    }
+    float cmax[NT];
+    bool need_any = false;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        cmax[nt] = score_max(sv[nt]);
+        need_any |= cmax[nt] > s.m[nt] + s.rowthr[nt];
+    }
+    if (__any(need_any)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const bool need = cmax[nt] > s.m[nt] + s.rowthr[nt];
+            const float mn = need ? cmax[nt] : s.m[nt];
+            const float alpha = need ? __builtin_amdgcn_exp2f((s.m[nt] - mn) * s.rowmul[nt]) : 1.0f;
+#pragma unroll
+            for (int t = 0; t < D / 16; ++t) { s.O[nt][t] *= alpha; }
+            s.l[nt] *= alpha;
+            s.m[nt] = mn;
+        }
+    }
+}
+
+// O^T += V'^T P^T, l += ones x P^T.
+template <int D, bool BF, int NT>
+__device__ __forceinline__ void chunk_values(const char* buf, int ci, int c, int g, const float (&sv)[NT][8], PromptRows<D, BF, NT>& s) {
+    using PG = PromptGeo<D, BF, 1>;
+    u4 ph[NT], pl[NT]; // P^T operand: FP16, or two BF16 terms
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const float bias = s.m[nt] == -INFINITY ? 0.0f : fmaf(-s.m[nt], s.rowmul[nt], kPOffset);
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { p[i] = __builtin_amdgcn_exp2f(fmaf(sv[nt][i], s.rowmul[nt], bias)); }
+        if constexpr (BF) {
+            bf8 hi, lo;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                hi[i] = static_cast<__bf16>(p[i]);
+                lo[i] = static_cast<__bf16>(p[i] - static_cast<float>(hi[i]));
+            }
+            ph[nt] = __builtin_bit_cast(u4, hi);
+            pl[nt] = __builtin_bit_cast(u4, lo);
+        } else {
+            h8 x;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { x[i] = static_cast<_Float16>(p[i]); }
+            ph[nt] = __builtin_bit_cast(u4, x);
+        }
+    }
+    const char* vp = buf + PG::kPlane + c * PG::kRowV;
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+        const u4 va = *reinterpret_cast<const u4*>(vp + 16 * t * PG::kRowV + 16 * v_slot<D>(4 * ci + g, 16 * t + c));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            if constexpr (BF) {
+                s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, va), __builtin_bit_cast(bf8, ph[nt]), s.O[nt][t], 0, 0, 0);
+                s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, va), __builtin_bit_cast(bf8, pl[nt]), s.O[nt][t], 0, 0, 0);
+            } else {
+                s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va), __builtin_bit_cast(h8, ph[nt]), s.O[nt][t], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        if constexpr (BF) {
+            bf8 ones;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { ones[i] = static_cast<__bf16>(1.0f); }
+            s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(bf8, ph[nt]), s.l[nt], 0, 0, 0);
+            s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(bf8, pl[nt]), s.l[nt], 0, 0, 0);
+        } else {
+            const h8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
+            s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, __builtin_bit_cast(h8, ph[nt]), s.l[nt], 0, 0, 0);
+        }
+    }
+}
+
+// ---- tiles that need care ------------------------------------------------------------------------
+//
+// The FP16 operands K' and V' cannot hold a code times a scale of 512 or more, and a masked key's zero
+// probability times an infinite V is NaN on the matrix cores. Both are rare (outliers of a cache), so the loop over
+// the tiles only notices them; a workgroup that did walks its keys once more, with the forms below in the
+// tiles that have such values.
+// One K group of scale 600 in the history, 512 tokens at 40/8/128 on MI355X: over 2,000 rows 191 us (64 without it;
+// verify launches 1,040, whose merge computes the group's split again), over 8,000 rows 439 (180; 2,975).
+
+// S^T of one 32-key chunk with FP32 operands: FP32(code) * scale (reference decode
+// include/ninfer/ops/gqa_attention.h:30), q in FP32 in the units of the wave's FP16 operand.
+template <int D, int NT>
+__device__ __forceinline__ void scores_f32(const PromptArgs& a, const HeadPlanes<D, false>& hp, int h, int c0, int row0, int rows, int c, int g,
+                                           const float (&rowmul)[NT], f4 (&sacc)[2][NT]) {
+    const uint16_t* src[NT];
+    float factor[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int r = min(row0 + 16 * nt + c, rows - 1); // rows past the end are masked
+        const int t = r / a.G;
+        src[nt] = a.q + static_cast<int64_t>(D) * (h * a.G + (r - t * a.G) + static_cast<int64_t>(a.Hq) * t);
+        factor[nt] = a.scale_log2 / rowmul[nt]; // an exact power of two
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) { sacc[kt][nt] = f4{0.f, 0.f, 0.f, 0.f}; }
+    }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+        const int key = c0 + 16 * kt + c;
+#pragma unroll 1
+        for (int ks = 0; ks < D / 32; ++ks) {
+            const int d0 = 8 * (4 * ks + g);
+            const u2 code = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(hp.k, key * D + d0, 0, 0));
+            const float sc = f16_bits_to_f32(__builtin_amdgcn_raw_buffer_load_b16(hp.ks, 2 * (key * (D / 64) + d0 / 64), 0, 0));
+            u4 q[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) { q[nt] = *reinterpret_cast<const u4*>(src[nt] + d0); }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float k = static_cast<float>(static_cast<int8_t>(code[e >> 2] >> (8 * (e & 3)))) * sc;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const float x = __uint_as_float((e & 1) ? q[nt][e >> 1] & 0xffff0000u : q[nt][e >> 1] << 16) * factor[nt];
+                    sacc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, x, sacc[kt][nt], 0, 0, 0);
+                }
+            }
+        }
+    }
+}
+
+// Four V values (dims d0 .. d0 + 3) of a key, in FP32.
+template <int D, bool BF>
+__device__ __forceinline__ f4 v_values(const HeadPlanes<D, BF>& hp, int key, int d0) {
+    if constexpr (BF) {
+        const u2 w = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(hp.v, 2 * (key * D + d0), 0, 0));
+        return f4{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16),
+                  __uint_as_float(w[1] & 0xffff0000u)};
+    } else {
+        const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(hp.v, key * D + d0, 0, 0);
+        const float sc = f16_bits_to_f32(__builtin_amdgcn_raw_buffer_load_b16(hp.vs, 2 * (key * (D / 64) + d0 / 64), 0, 0));
+        return f4{static_cast<float>(static_cast<int8_t>(w)), static_cast<float>(static_cast<int8_t>(w >> 8)),
+                  static_cast<float>(static_cast<int8_t>(w >> 16)), static_cast<float>(static_cast<int8_t>(w >> 24))} * sc;
+    }
+}
+
+// O^T += V^T P^T of one chunk with FP32 operands (infinite and NaN values left out), l += sum of P.
+// p[nt][i] of lane (c, g): key c0 + 16 (i >> 2) + 4g + (i & 3) of row 16nt + c, which is the B operand of step i.
+template <int D, int NT>
+__device__ __forceinline__ void values_f32(const HeadPlanes<D, false>& hp, int c0, int c, int g, const float (&p)[NT][8],
+                                           f4 (&O)[NT][D / 16], f4 (&l)[NT]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int key = c0 + 16 * (i >> 2) + 4 * g + (i & 3);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) { l[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(1.0f, p[nt][i], l[nt], 0, 0, 0); }
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) {
+            if (t % 4 == 0) { __builtin_amdgcn_sched_barrier(0); } // few loads at once: the state fills the registers
+            const int d = 16 * t + c;
+            const float code = static_cast<float>(static_cast<int8_t>(__builtin_amdgcn_raw_buffer_load_b8(hp.v, key * D + d, 0, 0)));
+            const float v = code * f16_bits_to_f32(__builtin_amdgcn_raw_buffer_load_b16(hp.vs, 2 * (key * (D / 64) + d / 64), 0, 0));
+            const float x = __builtin_isfinite(v) ? v : 0.0f;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) { O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, p[nt][i], O[nt][t], 0, 0, 0); }
+        }
+    }
+}
+
+// A chunk's probabilities in FP32.
+template <int D, bool BF, int NT>
+__device__ __forceinline__ void chunk_probabilities(const float (&sv)[NT][8], const PromptRows<D, BF, NT>& s, float (&p)[NT][8]) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            p[nt][i] = s.m[nt] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(sv[nt][i] - s.m[nt], s.rowmul[nt], kPOffset));
+        }
+    }
+}
+
+// The infinite and NaN V values of a chunk, to the rows that give their key a probability above zero only.
+template <int D, bool BF, int NT>
+__device__ __forceinline__ void add_nonfinite(const HeadPlanes<D, BF>& hp, int c0, int window, int c, int g, const float (&p)[NT][8],
+                                              f4 (&O)[NT][D / 16]) {
+#pragma unroll 1
+    for (int kk = 0; kk < 32; ++kk) {
+        const int key = c0 + kk;
+        if (key >= window) { break; }
+        bool any = false;
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) {
+            if (t % 4 == 0) { __builtin_amdgcn_sched_barrier(0); }
+            const f4 v = v_values<D, BF>(hp, key, 16 * t + 4 * g);
+            any |= !(__builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]));
+        }
+        if (!__any(any)) { continue; }
+        const int i = 4 * (kk >> 4) + (kk & 3);
+        const int from = 16 * ((kk >> 2) & 3) + c;
+        float pk[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            float x = p[nt][0];
+#pragma unroll
+            for (int e = 1; e < 8; ++e) { x = i == e ? p[nt][e] : x; }
+            pk[nt] = __shfl(x, from, 64);
+        }
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) {
+            if (t % 4 == 0) { __builtin_amdgcn_sched_barrier(0); }
+            const f4 v = v_values<D, BF>(hp, key, 16 * t + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (__builtin_isfinite(v[e])) { continue; }
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    if (pk[nt] != 0.0f) { O[nt][t][e] = fmaf(pk[nt], v[e], O[nt][t][e]); }
+                }
+            }
+        }
+    }
+}
+
+// A workgroup's part: one row tile of one KV head over one key split. CARE: the walk with the forms above.
+// Returns whether this thread saw a value that needs it: a live INT8 scale of 512 or more.
+template <int D, bool BF, int WK, bool CARE>
+__device__ __forceinline__ bool prompt_tile(const PromptArgs& a, char* smem) {
     using PG = PromptGeo<D, BF, WK>;
     constexpr int NT = PG::NT;
     constexpr int KT = PG::KT;
-    __shared__ __attribute__((aligned(16))) char smem[PG::kSmem];
-    int* flag = reinterpret_cast<int*>(smem + 2 * PG::kBuf);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -357,8 +543,6 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
     const int tile = a.tiles - 1 - unit / a.nsplit;
     const int rows = a.T * a.G; // of this KV head
     const int r0 = tile * PG::BM;
-    if (tid == 0) { *flag = 0; }
-
     HeadPlanes<D, BF> hp;
     {
         const int64_t plane = static_cast<int64_t>(a.P) * D;
@@ -375,7 +559,7 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
     // The first key tile of an unsplit row tile does not depend on the positions: its loads (inside the
     // padded cache) go out before them.
     TileRegs<D, BF> tr;
-    if (a.nsplit == 1) { load_tile<D, BF>(hp, 0, tid, tr); }
+    if (!CARE && a.nsplit == 1) { load_tile<D, BF>(hp, 0, tid, tr); }
     const int window = max(0, min(a.positions[a.T - 1] + 1, a.max_keys));
     const int t_last = (min(r0 + PG::BM, rows) - 1) / a.G;
     const int kend = min(window, a.positions[t_last] + 1); // keys any row of the tile sees
@@ -383,7 +567,7 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
     const int per = (ntile + a.nsplit - 1) / a.nsplit;
     const int j0 = split * per;
     ntile = min(ntile, j0 + per); // key tiles [j0, ntile) are this workgroup's
-    if (a.nsplit > 1 && j0 < ntile) { load_tile<D, BF>(hp, j0 * KT, tid, tr); }
+    if (!CARE && a.nsplit > 1 && j0 < ntile) { load_tile<D, BF>(hp, j0 * KT, tid, tr); }
 
     // ---- the wave's rows: Q operand, positions, softmax state
     PromptRows<D, BF, NT> s;
@@ -448,131 +632,81 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
     wave_min = __builtin_amdgcn_readfirstlane(wave_min);
     wave_max_pos = __builtin_amdgcn_readfirstlane(wave_max_pos);
 
-    uint32_t wide = 0u;
-    if (ntile > j0) { wide |= store_tile<D, BF>(tr, smem + (j0 & 1) * PG::kBuf, j0 * KT, window, tid); }
-    if (ntile > j0 + 1) { load_tile<D, BF>(hp, (j0 + 1) * KT, tid, tr); }
-    __syncthreads();
-
+    u16x2 top_scale = {0, 0};
+    if constexpr (!CARE) {
+        if (ntile > j0) { store_tile<D, BF>(tr, smem + (j0 & 1) * PG::kBuf, j0 * KT, window, tid, top_scale); }
+        if (ntile > j0 + 1) { load_tile<D, BF>(hp, (j0 + 1) * KT, tid, tr); }
+        __syncthreads();
 #pragma unroll 1
-    for (int j = j0; j < ntile; ++j) {
-        const char* buf = smem + (j & 1) * PG::kBuf;
-        if (j + 1 < ntile) {
-            wide |= store_tile<D, BF>(tr, smem + ((j + 1) & 1) * PG::kBuf, (j + 1) * KT, window, tid);
-            if (j + 2 < ntile) { load_tile<D, BF>(hp, (j + 2) * KT, tid, tr); }
+        for (int j = j0; j < ntile; ++j) {
+            const char* buf = smem + (j & 1) * PG::kBuf;
+            if (j + 1 < ntile) {
+                store_tile<D, BF>(tr, smem + ((j + 1) & 1) * PG::kBuf, (j + 1) * KT, window, tid, top_scale);
+                if (j + 2 < ntile) { load_tile<D, BF>(hp, (j + 2) * KT, tid, tr); }
+            }
+#pragma unroll
+            for (int cw = 0; cw < PG::NCH / WK; ++cw) {
+                const int ci = cw * WK + wk;
+                const int c0 = j * KT + 32 * ci;
+                if (c0 > wave_max_pos) { continue; }
+                f4 sacc[2][NT];
+                float sv[NT][8];
+                chunk_scores<D, BF, NT>(buf, ci, c, g, s, sacc);
+                chunk_rescale<D, BF, NT>(sacc, c0, c0 + 31 > wave_min, g, s, sv);
+                chunk_values<D, BF, NT>(buf, ci, c, g, sv, s);
+            }
+            __syncthreads(); // buf is free, the next tile is in place
         }
-#pragma unroll
-        for (int cw = 0; cw < PG::NCH / WK; ++cw) {
-            const int ci = cw * WK + wk;
-            const int c0 = j * KT + 32 * ci;
-            if (c0 > wave_max_pos) { continue; }
-            // S^T = K' Q^T
-            f4 sacc[2][NT];
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                const char* krow = buf + (32 * ci + 16 * kt + c) * PG::kRowK;
-#pragma unroll
-                for (int ks = 0; ks < D / 32; ++ks) {
-                    const u4 ka = *reinterpret_cast<const u4*>(krow + 16 * ((4 * ks + g) ^ c));
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        const f4 acc = ks == 0 ? f4{0.f, 0.f, 0.f, 0.f} : sacc[kt][nt];
-                        if constexpr (BF) {
-                            sacc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, ka), __builtin_bit_cast(bf8, s.q[nt][ks]), acc, 0, 0, 0);
-                        } else {
-                            sacc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, ka), __builtin_bit_cast(h8, s.q[nt][ks]), acc, 0, 0, 0);
-                        }
+    } else {
+        // bit j - j0: tile j needs care
+        uint32_t* marks = reinterpret_cast<uint32_t*>(smem + 2 * PG::kBuf);
+        for (int i = tid; 32 * i < ntile - j0; i += kPromptThreads) { marks[i] = 0u; }
+        __syncthreads();
+#pragma unroll 1
+        for (int j = j0; j < ntile; ++j) {
+            load_tile<D, BF>(hp, j * KT, tid, tr);
+            bool mark = false;
+            top_scale = u16x2{0, 0};
+            store_tile<D, BF>(tr, smem, j * KT, window, tid, top_scale);
+            mark |= wide_scale(top_scale);
+            if (mark) { atomicOr(&marks[(j - j0) >> 5], 1u << ((j - j0) & 31)); }
+            __syncthreads();
+            const bool care = ((marks[(j - j0) >> 5] >> ((j - j0) & 31)) & 1u) != 0u;
+#pragma unroll 1
+            for (int cw = 0; cw < PG::NCH / WK; ++cw) {
+                const int ci = cw * WK + wk;
+                const int c0 = j * KT + 32 * ci;
+                if (c0 > wave_max_pos || (!BF && care)) { continue; }
+                f4 sacc[2][NT];
+                float sv[NT][8];
+                chunk_scores<D, BF, NT>(smem, ci, c, g, s, sacc);
+                chunk_rescale<D, BF, NT>(sacc, c0, true, g, s, sv);
+                chunk_values<D, BF, NT>(smem, ci, c, g, sv, s);
+            }
+            __syncthreads();
+        }
+        if constexpr (!BF) { // the marked tiles (a softmax takes its keys in any order)
+#pragma unroll 1
+            for (int base = 0; base < ntile - j0; base += 32) {
+                uint32_t bits = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(marks[base >> 5])));
+#pragma unroll 1
+                for (; bits != 0u; bits &= bits - 1u) {
+                    const int j = j0 + base + __builtin_ctz(bits);
+#pragma unroll 1
+                    for (int cw = 0; cw < PG::NCH / WK; ++cw) {
+                        const int c0 = j * KT + 32 * (cw * WK + wk);
+                        if (c0 > wave_max_pos) { continue; }
+                        f4 sacc[2][NT];
+                        float sv[NT][8], p[NT][8];
+                        scores_f32<D, NT>(a, hp, h, c0, r0 + 16 * NT * wr, rows, c, g, s.rowmul, sacc);
+                        chunk_rescale<D, BF, NT>(sacc, c0, true, g, s, sv);
+                        chunk_probabilities<D, BF, NT>(sv, s, p);
+                        values_f32<D, NT>(hp, c0, c, g, p, s.O, s.l);
+                        add_nonfinite<D, BF, NT>(hp, c0, window, c, g, p, s.O);
                     }
-                }
-            }
-            // lazy online softmax (constants and rounding as in verify_attention.hip)
-            float sv[NT][8];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) { sv[nt][i] = sacc[i >> 2][nt][i & 3]; }
-            }
-            if (c0 + 31 > wave_min) {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const int key = c0 + 16 * (i >> 2) + 4 * g + (i & 3);
-                        sv[nt][i] = key <= s.pos[nt] ? sv[nt][i] : -INFINITY;
-                    }
-                }
-            }
-            float cmax[NT];
-            bool need_any = false;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                cmax[nt] = score_max(sv[nt]);
-                need_any |= cmax[nt] > s.m[nt] + s.rowthr[nt];
-            }
-            if (__any(need_any)) {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const bool need = cmax[nt] > s.m[nt] + s.rowthr[nt];
-                    const float mn = need ? cmax[nt] : s.m[nt];
-                    const float alpha = need ? __builtin_amdgcn_exp2f((s.m[nt] - mn) * s.rowmul[nt]) : 1.0f;
-#pragma unroll
-                    for (int t = 0; t < D / 16; ++t) { s.O[nt][t] *= alpha; }
-                    s.l[nt] *= alpha;
-                    s.m[nt] = mn;
-                }
-            }
-            u4 ph[NT], pl[NT]; // P^T operand: FP16, or two BF16 terms
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const float bias = s.m[nt] == -INFINITY ? 0.0f : fmaf(-s.m[nt], s.rowmul[nt], kPOffset);
-                float p[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) { p[i] = __builtin_amdgcn_exp2f(fmaf(sv[nt][i], s.rowmul[nt], bias)); }
-                if constexpr (BF) {
-                    bf8 hi, lo;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        hi[i] = static_cast<__bf16>(p[i]);
-                        lo[i] = static_cast<__bf16>(p[i] - static_cast<float>(hi[i]));
-                    }
-                    ph[nt] = __builtin_bit_cast(u4, hi);
-                    pl[nt] = __builtin_bit_cast(u4, lo);
-                } else {
-                    h8 x;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) { x[i] = static_cast<_Float16>(p[i]); }
-                    ph[nt] = __builtin_bit_cast(u4, x);
-                }
-            }
-            // O^T += V'^T P^T, l += ones x P^T
-            const char* vp = buf + PG::kPlane + c * PG::kRowV;
-#pragma unroll
-            for (int t = 0; t < D / 16; ++t) {
-                const u4 va = *reinterpret_cast<const u4*>(vp + 16 * t * PG::kRowV + 16 * v_slot<D>(4 * ci + g, 16 * t + c));
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    if constexpr (BF) {
-                        s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, va), __builtin_bit_cast(bf8, ph[nt]), s.O[nt][t], 0, 0, 0);
-                        s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, va), __builtin_bit_cast(bf8, pl[nt]), s.O[nt][t], 0, 0, 0);
-                    } else {
-                        s.O[nt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va), __builtin_bit_cast(h8, ph[nt]), s.O[nt][t], 0, 0, 0);
-                    }
-                }
-            }
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                if constexpr (BF) {
-                    bf8 ones;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) { ones[i] = static_cast<__bf16>(1.0f); }
-                    s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(bf8, ph[nt]), s.l[nt], 0, 0, 0);
-                    s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(bf8, pl[nt]), s.l[nt], 0, 0, 0);
-                } else {
-                    const h8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
-                    s.l[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, __builtin_bit_cast(h8, ph[nt]), s.l[nt], 0, 0, 0);
                 }
             }
         }
-        __syncthreads(); // buf is free, the next tile is in place
     }
 
     // ---- merge the WK key waves of each row tile through LDS, or take the one wave's rows as they are
@@ -630,32 +764,38 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
             }
         }
     }
-    bool bad = false;
+    bool again = !CARE && wide_scale(top_scale);
     const int64_t part = ((static_cast<int64_t>(tile) * a.Hkv + h) * a.nsplit + split) * PG::BM; // first partial row
     if (wk == 0) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const int rr = 16 * (NT * wr + nt) + c; // row within the tile
             const int r = r0 + rr;
-            const int t = r / a.G;
-            const int gi = r - t * a.G;
             const float inv = L[nt] > 0.0f ? 1.0f / L[nt] : 0.0f;
-            bad |= !__builtin_isfinite(L[nt]);
-            const int64_t orow = static_cast<int64_t>(D) * (h * a.G + gi + static_cast<int64_t>(a.Hq) * t);
 #pragma unroll
             for (int t8 = 0; t8 < D / 16; ++t8) {
-                const f4 o = L[nt] > 0.0f ? s.O[nt][t8] * inv : f4{0.f, 0.f, 0.f, 0.f};
-                const int d = 16 * t8 + 4 * g;
-                bad |= !(__builtin_isfinite(o[0]) && __builtin_isfinite(o[1]) && __builtin_isfinite(o[2]) && __builtin_isfinite(o[3]));
-                if (a.nsplit > 1) {
-                    *reinterpret_cast<u2*>(a.part_o + (part + rr) * D + d) =
+                s.O[nt][t8] = L[nt] > 0.0f ? s.O[nt][t8] * inv : f4{0.f, 0.f, 0.f, 0.f};
+            }
+            if (a.nsplit > 1) {
+                uint16_t* dst = a.part_o + (part + rr) * D + 4 * g;
+#pragma unroll
+                for (int t8 = 0; t8 < D / 16; ++t8) {
+                    const f4 o = s.O[nt][t8];
+                    *reinterpret_cast<u2*>(dst + 16 * t8) =
                         u2{static_cast<uint32_t>(f32_to_f16_bits(o[0])) | (static_cast<uint32_t>(f32_to_f16_bits(o[1])) << 16),
                            static_cast<uint32_t>(f32_to_f16_bits(o[2])) | (static_cast<uint32_t>(f32_to_f16_bits(o[3])) << 16)};
-                } else if (r < rows) {
-                    if (a.out_f32) {
-                        *reinterpret_cast<f4*>(static_cast<float*>(a.out) + orow + d) = o;
-                    } else {
-                        *reinterpret_cast<u2*>(static_cast<uint16_t*>(a.out) + orow + d) =
+                }
+            } else if (r < rows) {
+                const int t = r / a.G;
+                const int64_t first = static_cast<int64_t>(D) * (h * a.G + (r - t * a.G) + static_cast<int64_t>(a.Hq) * t) + 4 * g;
+                if (a.out_f32) {
+#pragma unroll
+                    for (int t8 = 0; t8 < D / 16; ++t8) { *reinterpret_cast<f4*>(static_cast<float*>(a.out) + first + 16 * t8) = s.O[nt][t8]; }
+                } else {
+#pragma unroll
+                    for (int t8 = 0; t8 < D / 16; ++t8) {
+                        const f4 o = s.O[nt][t8];
+                        *reinterpret_cast<u2*>(static_cast<uint16_t*>(a.out) + first + 16 * t8) =
                             u2{static_cast<uint32_t>(f32_to_bf16_bits(o[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[1])) << 16),
                                static_cast<uint32_t>(f32_to_bf16_bits(o[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[3])) << 16)};
                     }
@@ -663,32 +803,119 @@ __global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(
             }
         }
     }
-    // A K scale of 512 or more (FP16(code * scale) may overflow and drop a key silently), or a result
-    // the FP16 operands could not hold: the rows are computed again, exactly (here, or by the merge).
-    bool redo = false;
-    if constexpr (!BF) {
-        if (__any(bad || (wide & 0x4000u) != 0u) && lane == 0) { *flag = 1; }
-        __syncthreads();
-        redo = *flag != 0;
-    }
-    if (a.nsplit > 1) {
-        if (wk == 0 && g == 0) {
+    if (a.nsplit > 1 && wk == 0 && g == 0) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int64_t i = part + 16 * (NT * wr + nt) + c;
-                *reinterpret_cast<float2*>(a.part_ml + 2 * i) = float2{M[nt], redo ? -1.0f : L[nt]};
+        for (int nt = 0; nt < NT; ++nt) {
+            const int64_t i = part + 16 * (NT * wr + nt) + c;
+            *reinterpret_cast<float2*>(a.part_ml + 2 * i) = float2{M[nt], L[nt]};
+        }
+    }
+    return again;
+}
+
+template <int D, bool BF, int WK>
+__global__ __launch_bounds__(kPromptThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prompt_attn_kernel(PromptArgs a) {
+    using PG = PromptGeo<D, BF, WK>;
+    __shared__ __attribute__((aligned(16))) char smem[PG::kSmem];
+    int* flag = reinterpret_cast<int*>(smem + 2 * PG::kBuf);
+    if (threadIdx.x == 0) { *flag = 0; } // barriers below
+    if (prompt_tile<D, BF, WK, false>(a, smem)) { *flag = 1; }
+    __syncthreads();
+    if (__builtin_expect(*flag != 0, 0)) {
+        __syncthreads(); // the flag is read, the first walk's buffers are free
+        (void)prompt_tile<D, BF, WK, true>(a, smem);
+    }
+}
+
+// One row over the keys [k0, k1) in FP32 (the tiles' FP32 form), for a split whose O / l the FP16 partial
+// could not hold: the log2-domain maximum and the sum (with the partials' 2^kPOffset) to every thread, O to
+// xo[D]. Whole workgroup.
+constexpr int kExactFloats(int D) { return D + kPromptThreads + 16 + 4 * kPromptThreads; }
+
+template <int D>
+__device__ void exact_split_row(const PromptArgs& a, int h, int t, int qh, int k0, int k1, float* xs, float& M, float& L, const float*& xo) {
+    constexpr int GQ = D / 64;
+    constexpr int TPR = D / 4;                  // threads per V row
+    constexpr int PARTS = kPromptThreads / TPR; // key parts of a block
+    float* xq = xs;                    // [D] q * scale * log2(e)
+    float* xp = xs + D;                // probabilities of a block of keys
+    float* xr = xp + kPromptThreads;   // reductions
+    float* xv = xr + 16;               // [PARTS][D]
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int d4 = 4 * (tid % TPR);
+    const int part = tid / TPR;
+    const int64_t orow = static_cast<int64_t>(D) * (qh + static_cast<int64_t>(a.Hq) * t);
+    const int8_t* kbase = a.kc + static_cast<int64_t>(h) * a.P * D;
+    const int8_t* vbase = a.vc + static_cast<int64_t>(h) * a.P * D;
+    const uint16_t* ksb = a.ks + static_cast<int64_t>(h) * a.P * GQ;
+    const uint16_t* vsb = a.vs + static_cast<int64_t>(h) * a.P * GQ;
+    __syncthreads(); // the caller's use of xs is over
+    if (tid < D) { xq[tid] = bf16_to_f32(a.q[orow + tid]) * a.scale_log2; }
+    __syncthreads();
+    M = -INFINITY;
+    L = 0.0f;
+    f4 O = {0.f, 0.f, 0.f, 0.f};
+    for (int base = k0; base < k1; base += kPromptThreads) {
+        const int key = base + tid;
+        float sc = -INFINITY;
+        if (key < k1) {
+            sc = 0.0f;
+#pragma unroll
+            for (int gq = 0; gq < GQ; ++gq) {
+                const float ksc = f16_bits_to_f32(ksb[static_cast<int64_t>(key) * GQ + gq]);
+                u4 code[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { code[i] = *reinterpret_cast<const u4*>(kbase + static_cast<int64_t>(key) * D + 64 * gq + 16 * i); }
+                float p = 0.0f;
+#pragma unroll
+                for (int d = 0; d < 64; ++d) {
+                    p = fmaf(xq[64 * gq + d], static_cast<float>(static_cast<int8_t>(code[d >> 4][(d >> 2) & 3] >> (8 * (d & 3)))) * ksc, p);
+                }
+                sc += p;
             }
         }
-        return;
-    }
-    if constexpr (!BF) {
-        if (!redo) { return; }
-#pragma unroll 1
-        for (int r = r0; r < min(r0 + PG::BM, rows); ++r) {
-            const int t = r / a.G;
-            prompt_exact_row<D>(a, h, t, h * a.G + (r - t * a.G), min(a.positions[t], window - 1), reinterpret_cast<float*>(smem));
+        const float wm = wave_max(sc);
+        if (lane == 0) { xr[wave] = wm; }
+        __syncthreads();
+        float Mn = M;
+        for (int w = 0; w < kPromptThreads / 64; ++w) { Mn = fmaxf(Mn, xr[w]); }
+        const float alpha = (M == -INFINITY || Mn == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
+        const float p = (sc == -INFINITY || Mn == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(sc - Mn + kPOffset);
+        xp[tid] = p;
+        const float wsum = wave_sum(p);
+        if (lane == 0) { xr[8 + wave] = wsum; }
+        __syncthreads();
+        float bs = 0.0f;
+        for (int w = 0; w < kPromptThreads / 64; ++w) { bs += xr[8 + w]; }
+        L = fmaf(L, alpha, bs);
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+        for (int j = 0; j < kPromptThreads / PARTS; ++j) {
+            const int i = part * (kPromptThreads / PARTS) + j;
+            const int k = min(base + i, k1 - 1); // past the end: probability zero
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(vbase + static_cast<int64_t>(k) * D + d4);
+            const float vs = f16_bits_to_f32(vsb[static_cast<int64_t>(k) * GQ + d4 / 64]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = static_cast<float>(static_cast<int8_t>(w >> (8 * e))) * vs;
+                acc[e] = xp[i] != 0.0f ? fmaf(xp[i], x, acc[e]) : acc[e];
+            }
         }
+        O = O * alpha + acc;
+        M = Mn;
+        __syncthreads(); // xp and xr are reused
     }
+    *reinterpret_cast<f4*>(xv + part * D + d4) = O;
+    __syncthreads();
+    if (tid < D) {
+        float o = 0.0f;
+        for (int w = 0; w < PARTS; ++w) { o += xv[w * D + tid]; }
+        xp[tid] = o;
+    }
+    __syncthreads();
+    xo = xp;
 }
 
 // Log-sum-exp merge of a row's key splits: D / 4 threads per row, four dims each.
@@ -696,58 +923,99 @@ template <int D, bool BF>
 __global__ __launch_bounds__(kPromptThreads) void prompt_merge_kernel(PromptArgs a, int bm) {
     constexpr int TPR = D / 4;
     constexpr int RPB = kPromptThreads / TPR;
-    __shared__ float xs[D + 2 * kPromptThreads];
-    __shared__ int flag;
+    constexpr int KT = 16384 / D;
+    __shared__ __attribute__((aligned(16))) float xs[kExactFloats(D)];
+    __shared__ uint32_t redo[RPB]; // per row: the splits to compute again
     const int tid = threadIdx.x;
-    if (tid == 0) { flag = 0; }
+    if (tid < RPB) { redo[tid] = 0u; }
     __syncthreads();
     const int h = static_cast<int>(blockIdx.x) % a.Hkv;
     const int rb = static_cast<int>(blockIdx.x) / a.Hkv * RPB;
     const int rows = a.T * a.G;
     const int r = rb + tid / TPR;
     const int d = 4 * (tid % TPR);
-    bool bad = false;
+    float M = -INFINITY, L = 0.0f;
+    f4 O = {0.f, 0.f, 0.f, 0.f};
+    const auto add = [&](float m, float l, f4 o) { // o: O / l
+        const float Mn = fmaxf(M, m);
+        const float al = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
+        const float be = l * __builtin_amdgcn_exp2f(m - Mn);
+        O = O * al + o * be;
+        L = fmaf(L, al, be);
+        M = Mn;
+    };
     if (r < rows) {
         const int64_t first = ((static_cast<int64_t>(r / bm) * a.Hkv + h) * a.nsplit) * bm + r % bm;
-        float M = -INFINITY, L = 0.0f;
-        f4 O = {0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < a.nsplit; ++k) {
             const int64_t i = first + static_cast<int64_t>(k) * bm;
             const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * i);
             const u2 w = *reinterpret_cast<const u2*>(a.part_o + i * D + d);
-            bad |= ml.y < 0.0f;
             if (!(ml.y > 0.0f)) { continue; } // no visible key
             const f4 o = {f16_bits_to_f32(static_cast<uint16_t>(w[0])), f16_bits_to_f32(static_cast<uint16_t>(w[0] >> 16)),
                           f16_bits_to_f32(static_cast<uint16_t>(w[1])), f16_bits_to_f32(static_cast<uint16_t>(w[1] >> 16))};
-            bad |= !(__builtin_isfinite(o[0]) && __builtin_isfinite(o[1]) && __builtin_isfinite(o[2]) && __builtin_isfinite(o[3]));
-            const float Mn = fmaxf(M, ml.x);
-            const float al = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
-            const float be = ml.y * __builtin_amdgcn_exp2f(ml.x - Mn);
-            O = O * al + o * be;
-            L = fmaf(L, al, be);
-            M = Mn;
-        }
-        const f4 o = L > 0.0f ? O * (1.0f / L) : f4{0.f, 0.f, 0.f, 0.f};
-        const int t = r / a.G;
-        const int64_t orow = static_cast<int64_t>(D) * (h * a.G + (r - t * a.G) + static_cast<int64_t>(a.Hq) * t);
-        if (a.out_f32) {
-            *reinterpret_cast<f4*>(static_cast<float*>(a.out) + orow + d) = o;
-        } else {
-            *reinterpret_cast<u2*>(static_cast<uint16_t*>(a.out) + orow + d) =
-                u2{static_cast<uint32_t>(f32_to_bf16_bits(o[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[1])) << 16),
-                   static_cast<uint32_t>(f32_to_bf16_bits(o[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[3])) << 16)};
+            if constexpr (!BF) {
+                // O / l beyond FP16 (a V scale of 512 or more)
+                if (!(__builtin_isfinite(o[0]) && __builtin_isfinite(o[1]) && __builtin_isfinite(o[2]) && __builtin_isfinite(o[3]))) {
+                    atomicOr(&redo[tid / TPR], 1u << k);
+                }
+            }
+            add(ml.x, ml.y, o);
         }
     }
     if constexpr (!BF) {
-        if (__any(bad) && (tid & 63) == 0) { flag = 1; }
         __syncthreads();
-        if (flag == 0) { return; }
-        const int window = max(0, min(a.positions[a.T - 1] + 1, a.max_keys));
+        uint32_t any = 0u;
+        for (int i = 0; i < RPB; ++i) { any |= redo[i]; }
+        if (any != 0u) {
+            // a row with such a split is merged again in the same order, those splits in FP32
+            const int window = max(0, min(a.positions[a.T - 1] + 1, a.max_keys));
 #pragma unroll 1
-        for (int q = rb; q < min(rb + RPB, rows); ++q) {
-            const int t = q / a.G;
-            prompt_exact_row<D>(a, h, t, h * a.G + (q - t * a.G), min(a.positions[t], window - 1), xs);
+            for (int i = 0; i < RPB; ++i) {
+                const uint32_t again = redo[i];
+                if (again == 0u) { continue; }
+                const int rr = rb + i;
+                const int t = rr / a.G;
+                const int last = (min(rr / bm * bm + bm, rows) - 1) / a.G; // the row tile's last token bounds its key tiles
+                const int ntile = (max(min(window, a.positions[last] + 1), 0) + KT - 1) / KT;
+                const int per = (ntile + a.nsplit - 1) / a.nsplit;
+                const int seen = min(a.positions[t] + 1, window);
+                const bool mine = tid / TPR == i;
+                if (mine) {
+                    M = -INFINITY;
+                    L = 0.0f;
+                    O = f4{0.f, 0.f, 0.f, 0.f};
+                }
+                const int64_t first = ((static_cast<int64_t>(rr / bm) * a.Hkv + h) * a.nsplit) * bm + rr % bm;
+#pragma unroll 1
+                for (int k = 0; k < a.nsplit; ++k) {
+                    if ((again >> k) & 1u) {
+                        float m, l;
+                        const float* xo;
+                        exact_split_row<D>(a, h, t, h * a.G + (rr - t * a.G), k * per * KT, min((k + 1) * per * KT, seen), xs, m, l, xo);
+                        if (mine && l != 0.0f) { add(m, l, *reinterpret_cast<const f4*>(xo + d) * (1.0f / l)); }
+                    } else if (mine) {
+                        const int64_t at = first + static_cast<int64_t>(k) * bm;
+                        const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * at);
+                        const u2 w = *reinterpret_cast<const u2*>(a.part_o + at * D + d);
+                        if (ml.y != 0.0f) {
+                            add(ml.x, ml.y, f4{f16_bits_to_f32(static_cast<uint16_t>(w[0])), f16_bits_to_f32(static_cast<uint16_t>(w[0] >> 16)),
+                                               f16_bits_to_f32(static_cast<uint16_t>(w[1])), f16_bits_to_f32(static_cast<uint16_t>(w[1] >> 16))});
+                        }
+                    }
+                }
+            }
         }
+    }
+    if (r >= rows) { return; }
+    const f4 o = L > 0.0f ? O * (1.0f / L) : f4{0.f, 0.f, 0.f, 0.f};
+    const int t = r / a.G;
+    const int64_t orow = static_cast<int64_t>(D) * (h * a.G + (r - t * a.G) + static_cast<int64_t>(a.Hq) * t);
+    if (a.out_f32) {
+        *reinterpret_cast<f4*>(static_cast<float*>(a.out) + orow + d) = o;
+    } else {
+        *reinterpret_cast<u2*>(static_cast<uint16_t*>(a.out) + orow + d) =
+            u2{static_cast<uint32_t>(f32_to_bf16_bits(o[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[1])) << 16),
+               static_cast<uint32_t>(f32_to_bf16_bits(o[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(o[3])) << 16)};
     }
 }
 

@@ -69,6 +69,19 @@ def run_attention(case, out_f32=False, mode="A1", cache=None, stream=None, envel
     return res, cache
 
 
+def attention_us(case) -> float:
+    """Device time of one A1 call."""
+    D, Hq, Hkv, T, B = case.D, case.Hq, case.Hkv, case.T, case.B
+    cache = upload_cache(case)
+    dev = [DeviceArray.from_numpy(na.BF16, case.q, (D, Hq, T, B)), DeviceArray.from_numpy(na.BF16, case.k_new, (D, Hkv, T, B)),
+           DeviceArray.from_numpy(na.BF16, case.v_new, (D, Hkv, T, B)), DeviceArray.from_numpy(na.I32, case.positions, (T, B))]
+    out = DeviceArray(na.BF16, (D, Hq, T, B))
+    env = (min(case.Ls) + T, case.max_context)
+    ws = DeviceBuffer(ops.gqa_attention_workspace_bytes(Hq, Hkv, D, T, B, env[1]))
+    views, view, o = [x.tensor() for x in dev], cache.view(), out.tensor()
+    return time_us(lambda: ops.gqa_attention(*views, case.scale, view, env, ws, o))
+
+
 def append(case, cache, stream=None):
     D, Hkv, T, B = case.D, case.Hkv, case.T, case.B
     k = DeviceArray.from_numpy(na.BF16, case.k_new, (D, Hkv, T, B))

@@ -41,7 +41,7 @@ def test_tile_edges(gpu, Hq, Hkv, D, kv, L, T):
     _run(AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, kv=kv, seed=6000 + L + T + Hq))
 
 
-# A wide envelope (the plan follows its end, the keys the device positions) and one that clamps them.
+# A wide envelope: the plan follows its end, the keys the device positions.
 @pytest.mark.parametrize("L,T,cap", [(300, 70, 20000), (700, 300, 40000)])
 def test_wide_envelope(gpu, L, T, cap):
     print(f"case prompt envelope L={L} T={T} cap={cap}", flush=True)
@@ -63,6 +63,40 @@ def test_fp32_range(gpu, Hq, Hkv, D, L, T, absmax):
         for _ in range(6):
             sc[0, int(rng.integers(0, Hkv)), int(rng.integers(0, L)), int(rng.integers(0, D // 64))] = big
     _run(case)
+
+
+def _rare_scales(case, seed, n=6, absmax=1e5, planes=("ks", "vs")):
+    rng = np.random.default_rng(seed)
+    big = np.float16(absmax / 127.0).view(np.uint16)
+    for name in planes:
+        for _ in range(n):
+            getattr(case, name)[0, int(rng.integers(0, case.Hkv)), int(rng.integers(0, case.Ls[0])), int(rng.integers(0, case.D // 64))] = big
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,L,T", [
+    (40, 8, 128, 130, 1100), (40, 8, 128, 900, 300), (24, 4, 256, 100, 700), (16, 2, 256, 4000, 65), (40, 8, 128, 5000, 70)])
+@pytest.mark.parametrize("planes", [("ks",), ("vs",), ("ks", "vs")])
+def test_fp32_range_few_tiles(gpu, Hq, Hkv, D, L, T, planes):
+    """Such groups in a few key tiles among many, in each form of the kernel (256, 128 and 64 rows, one split and
+    several): only those tiles, and the partials that FP16 cannot hold, are computed in FP32."""
+    print(f"case prompt rare scales {Hq}/{Hkv}/{D} L={L} T={T} {planes}", flush=True)
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, seed=19, qstd=2e-5)
+    _rare_scales(case, L + T, planes=planes)
+    _run(case)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,L,T", [(40, 8, 128, 2000, 96), (40, 8, 128, 2000, 512), (24, 4, 256, 2000, 512)])
+@pytest.mark.parametrize("plane", ["ks", "vs"])
+def test_rare_scales_cost(gpu, Hq, Hkv, D, L, T, plane):
+    """One group beyond FP16's range costs its tile and the partials it reaches, not the whole prompt: at most 5 times
+    the plain prompt (MI355X: 3 times; a whole prompt computed again row by row took 57 to 250 times)."""
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, seed=4)
+    plain = gpu_runner.attention_us(case)
+    for h in range(Hkv):
+        getattr(case, plane)[0, h, 3, 0] = np.float16(600.0).view(np.uint16)
+    rare = gpu_runner.attention_us(case)
+    print(f"{Hq}/{Hkv}/{D} L={L} T={T} {plane}: {rare:.1f} us, plain {plain:.1f} us")
+    assert rare <= 5.0 * plain
 
 
 def test_unaligned_tensors_take_the_verify_launches(gpu):
