@@ -251,6 +251,25 @@ __device__ __forceinline__ void store_tile(const TileRegs<D, BF>& r, char* buf, 
 // A scale of 512 or more (an FP16 exponent of 24), NaN included.
 __device__ __forceinline__ bool wide_scale(u16x2 top) { return max(top.x, top.y) >= 0x6000; }
 
+// Zeros a thread's infinite and NaN BF16 V values of keys below `window`; returns whether there were any.
+template <int D>
+__device__ __forceinline__ bool drop_nonfinite(TileRegs<D, true>& r, int key0, int window, int tid) {
+    const int oct = tid / (D / 4);
+    const int kv0 = key0 + 32 * (oct >> 2) + 4 * (oct & 3);
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const uint32_t x = r.v[j][w];
+            const uint32_t bad = ((x & 0x7f807f80u) + 0x00800080u) & 0x80008000u; // an exponent of ones carries out
+            any |= bad != 0u && kv0 + (j & 3) + 16 * (j >> 2) < window;
+            r.v[j][w] = x & ~((bad >> 15) * 0xffffu);
+        }
+    }
+    return any;
+}
+
 // Online-softmax state of one wave.
 template <int D, bool BF, int NT>
 struct PromptRows {
@@ -524,7 +543,8 @@ __device__ __forceinline__ void add_nonfinite(const HeadPlanes<D, BF>& hp, int c
 }
 
 // A workgroup's part: one row tile of one KV head over one key split. CARE: the walk with the forms above.
-// Returns whether this thread saw a value that needs it: a live INT8 scale of 512 or more.
+// Returns whether this thread saw a value that needs it: a live INT8 scale of 512 or more, or a BF16 result that is
+// not finite.
 template <int D, bool BF, int WK, bool CARE>
 __device__ __forceinline__ bool prompt_tile(const PromptArgs& a, char* smem) {
     using PG = PromptGeo<D, BF, WK>;
@@ -666,6 +686,7 @@ __device__ __forceinline__ bool prompt_tile(const PromptArgs& a, char* smem) {
         for (int j = j0; j < ntile; ++j) {
             load_tile<D, BF>(hp, j * KT, tid, tr);
             bool mark = false;
+            if constexpr (BF) { mark = drop_nonfinite<D>(tr, j * KT, window, tid); }
             top_scale = u16x2{0, 0};
             store_tile<D, BF>(tr, smem, j * KT, window, tid, top_scale);
             mark |= wide_scale(top_scale);
@@ -682,6 +703,13 @@ __device__ __forceinline__ bool prompt_tile(const PromptArgs& a, char* smem) {
                 chunk_scores<D, BF, NT>(smem, ci, c, g, s, sacc);
                 chunk_rescale<D, BF, NT>(sacc, c0, true, g, s, sv);
                 chunk_values<D, BF, NT>(smem, ci, c, g, sv, s);
+                if constexpr (BF) {
+                    if (care) {
+                        float p[NT][8];
+                        chunk_probabilities<D, BF, NT>(sv, s, p);
+                        add_nonfinite<D, BF, NT>(hp, c0, window, c, g, p, s.O);
+                    }
+                }
             }
             __syncthreads();
         }
@@ -772,10 +800,16 @@ __device__ __forceinline__ bool prompt_tile(const PromptArgs& a, char* smem) {
             const int rr = 16 * (NT * wr + nt) + c; // row within the tile
             const int r = r0 + rr;
             const float inv = L[nt] > 0.0f ? 1.0f / L[nt] : 0.0f;
+            uint32_t top = 0u; // the largest magnitude's bits, doubled
 #pragma unroll
             for (int t8 = 0; t8 < D / 16; ++t8) {
                 s.O[nt][t8] = L[nt] > 0.0f ? s.O[nt][t8] * inv : f4{0.f, 0.f, 0.f, 0.f};
+                if constexpr (BF && !CARE) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { top = max(top, __float_as_uint(s.O[nt][t8][e]) << 1); }
+                }
             }
+            again |= top >= 0xff000000u;
             if (a.nsplit > 1) {
                 uint16_t* dst = a.part_o + (part + rr) * D + 4 * g;
 #pragma unroll

@@ -99,6 +99,31 @@ def test_rare_scales_cost(gpu, Hq, Hkv, D, L, T, plane):
     assert rare <= 5.0 * plain
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,kv,L,T", [(40, 8, 128, "bf16", 0, 100), (40, 8, 128, "bf16", 300, 600), (40, 8, 128, "bf16", 2500, 65),
+                                             (24, 4, 256, "bf16", 20, 300), (40, 8, 128, "i8", 10, 200), (16, 2, 256, "i8", 1500, 70)])
+@pytest.mark.parametrize("bits", [0x7F80, 0x7FC0])
+def test_non_finite_value_leaves_earlier_outputs(gpu, Hq, Hkv, D, kv, L, T, bits):
+    """An infinite or NaN V value reaches the outputs of the tokens that see it and no others."""
+    print(f"case prompt non-finite {Hq}/{Hkv}/{D} {kv} L={L} T={T} {bits:#x}", flush=True)
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, kv=kv, seed=33)
+    (planes, ref), at, head = case.oracle_after_append(), T // 2, 1
+    cache = gpu_runner.upload_cache(case)
+    gpu_runner.append(case, cache)
+    dirty = [x.copy() for x in planes]
+    if kv == "bf16":
+        dirty[1][0, head, L + at, 7] = bits
+    else:  # the scale of a group: FP16 infinity or NaN
+        dirty[3][0, head, L + at, 0] = 0x7C00 if bits == 0x7F80 else 0x7E00
+    cache.upload(*dirty)
+    out, _ = gpu_runner.run_attention(case, out_f32=True, mode="A3", cache=cache)
+    out, ref = np.asarray(out, np.float64).reshape(T, Hq, D), np.asarray(ref, np.float64).reshape(T, Hq, D)
+    G = Hq // Hkv
+    reached = np.zeros(out.shape, bool)
+    reached[at:, head * G:(head + 1) * G, (7 if kv == "bf16" else slice(0, 64))] = True
+    assert np.all(np.isfinite(out[~reached])) and rel_l2(out[~reached], ref[~reached]) <= REL_L2_F32
+    assert not np.any(np.isfinite(out[reached]))
+
+
 def test_unaligned_tensors_take_the_verify_launches(gpu):
     """q one element into its buffer: accepted as before, and within the same bar."""
     case = AttnCase([200], T=70, seed=17)
