@@ -984,7 +984,7 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_merge_kernel(PromptArgs
             const int64_t i = first + static_cast<int64_t>(k) * bm;
             const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * i);
             const u2 w = *reinterpret_cast<const u2*>(a.part_o + i * D + d);
-            if (!(ml.y > 0.0f)) { continue; } // no visible key
+            if (ml.y == 0.0f) { continue; } // no visible key (a NaN sum stays: the row's output is 0, as without splits)
             const f4 o = {f16_bits_to_f32(static_cast<uint16_t>(w[0])), f16_bits_to_f32(static_cast<uint16_t>(w[0] >> 16)),
                           f16_bits_to_f32(static_cast<uint16_t>(w[1])), f16_bits_to_f32(static_cast<uint16_t>(w[1] >> 16))};
             if constexpr (!BF) {

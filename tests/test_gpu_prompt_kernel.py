@@ -124,6 +124,25 @@ def test_non_finite_value_leaves_earlier_outputs(gpu, Hq, Hkv, D, kv, L, T, bits
     assert not np.any(np.isfinite(out[reached]))
 
 
+@pytest.mark.parametrize("L,T", [(100, 200), (2500, 65)])
+def test_nan_key_is_not_dropped(gpu, L, T):
+    """A row that sees a NaN key has no defined sum: it is 0 with one key split and with several, never the result
+    of the other splits alone."""
+    print(f"case prompt NaN key L={L} T={T}", flush=True)
+    case = AttnCase([L], T=T, kv="bf16", seed=35)
+    (planes, ref), head = case.oracle_after_append(), 2
+    cache = gpu_runner.upload_cache(case)
+    gpu_runner.append(case, cache)
+    dirty = [x.copy() for x in planes]
+    dirty[0][0, head, 40, 3] = 0x7FC0
+    cache.upload(*dirty)
+    out, _ = gpu_runner.run_attention(case, out_f32=True, mode="A3", cache=cache)
+    out, ref = np.asarray(out).reshape(T, 8, 5, 128), np.asarray(ref, np.float64).reshape(T, 8, 5, 128)
+    others = [h for h in range(8) if h != head]
+    assert rel_l2(out[:, others], ref[:, others]) <= REL_L2_F32
+    assert not np.any(out[:, head])
+
+
 def test_unaligned_tensors_take_the_verify_launches(gpu):
     """q one element into its buffer: accepted as before, and within the same bar."""
     case = AttnCase([200], T=70, seed=17)
