@@ -103,6 +103,9 @@ __device__ __forceinline__ float partial_o_at(const uint16_t* base, int64_t i) {
 }
 
 constexpr int kXcds = 8; // each with an L2 of its own
+// Shorter windows read too little to gain from it (16/2/256 on MI355X, T = 16: 2,116 keys 21.1 -> 21.5 us, 4,516 keys
+// 21.6 -> 21.95, 8,516 keys 26.5 -> 24.5).
+constexpr uint32_t kInterleavedKeys = 8192;
 
 struct AttnArgs {
     const uint16_t* q;
@@ -137,7 +140,6 @@ struct AttnArgs {
     float scale_log2; // softmax scale * log2(e)
     void* out;        // unsplit windows (DIRECT kernels): the rows' outputs, BF16 or FP32
     int32_t out_f32;
-    int32_t interleaved; // B == 1, BF16 cache of head_dim 256: one-dimensional grid of interleaved_part
 };
 
 // Keys per split of a batch-1 plan chosen on the device from the actual window, over the `launched`
@@ -1602,8 +1604,8 @@ __device__ __forceinline__ void pv_chunk_b(const float (&p)[NT][8], const ChunkR
 // Several row chunks at batch 1: each (KV head, split) has a workgroup per row chunk, all streaming the same keys,
 // and workgroups go to the 8 XCDs in turn. Where KV heads x splits is a multiple of 8 the grid (KV head, split, row
 // chunk) puts those workgroups on one XCD, whose L2 serves all but the first; elsewhere they are numbered 8
-// apart in a one-dimensional grid. MI355X, 24/4/256 over 32,774 keys, T = 6 (29 splits): 51.6 -> 40.6 us;
-// 190,000 keys 150 -> 148 us.
+// apart in a one-dimensional grid. MI355X, 24/4/256 over 32,774 keys, T = 6 (29 splits): 50.6 -> 36.7 us;
+// 16/2/256, T = 16: 32,784 keys 52.1 -> 38.5 us, 65,552 keys 93.0 -> 56.9.
 // The INT8 kernel is not bound by these reads and was 4 to 13% slower numbered so. Returns whether the
 // workgroup has a part.
 __device__ __forceinline__ bool interleaved_part(const AttnArgs& a, int& h, int& split, int& rc) {
@@ -1618,7 +1620,9 @@ __device__ __forceinline__ bool interleaved_part(const AttnArgs& a, int& h, int&
 }
 
 // DIRECT: one workgroup holds the whole window and writes the output (as verify_attn_direct_kernel).
-template <int NT, int D, bool ONCE, bool DIRECT = false>
+// INTERLEAVED: the one-dimensional grid of interleaved_part (an instance of its own: as a branch it cost the other
+// launches of several row chunks 1%).
+template <int NT, int D, bool ONCE, bool DIRECT = false, bool INTERLEAVED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void verify_attn_partial_bf16_kernel(AttnArgs a) {
     using GB = GeoB<D>;
     __shared__ __attribute__((aligned(16))) char smem[GB::kSmemBytes];
@@ -1632,8 +1636,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     int rc = blockIdx.z;
     int b = 0;
     int split = a.B == 1 ? blockIdx.y : blockIdx.x;
-    if constexpr (D == 256 && !ONCE && !DIRECT) {
-        if (a.interleaved != 0 && !interleaved_part(a, h, split, rc)) { return; }
+    if constexpr (INTERLEAVED) {
+        if (!interleaved_part(a, h, split, rc)) { return; }
     }
     int kps = a.kps;
     int slot0 = 0;
@@ -2700,14 +2704,18 @@ void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uin
     const bool dev = plan.b1_device_plan;
     if (c.kb != nullptr) {
         if (c.B == 1) { grid = grid_b1; }
-        // Short windows read too little to gain (704 keys 19.3 against 19.5 us, 2,106 keys 19.9 against 19.7), and
-        // head_dim 128 runs two workgroups per CU (T = 16 over 21,500 keys: 53.6 against 54.5 us).
+        // Interleaved, an XCD takes whole units of row_chunks workgroups; where that gives some XCD more rounds of its
+        // CUs than the grid needs, the plain numbering stays (24/4/256, T = 32 in 36 units of 7: 26.4 us against 33.8).
+        // Head_dim 128 runs two workgroups per CU (T = 16 over 21,500 keys: 53.6 plain, 54.5 us interleaved).
         const int units = c.Hkv * plan.split_slots;
-        if (c.B == 1 && c.D == 256 && !once && max_keys > 2048 && units % kXcds != 0) {
-            a.interleaved = 1;
+        constexpr int kCus = kAttnTargetWorkgroups / 2;
+        const auto rounds = [](int workgroups, int cus) { return (workgroups + cus - 1) / cus; };
+        const bool even = rounds((units + kXcds - 1) / kXcds * plan.row_chunks, kCus / kXcds) <= rounds(units * plan.row_chunks, kCus);
+        if (c.B == 1 && c.D == 256 && !once && max_keys > kInterleavedKeys && units % kXcds != 0 && even) {
             grid = dim3((units + kXcds - 1) / kXcds * kXcds * plan.row_chunks);
-        }
-        if (c.D == 128) {
+            // a row chunk of several holds more than 16 rows
+            hipLaunchKernelGGL((verify_attn_partial_bf16_kernel<2, 256, false, false, true>), grid, dim3(256), 0, stream, a);
+        } else if (c.D == 128) {
             if (rows <= 16) {
                 NMI_PARTIAL(verify_attn_partial_bf16_kernel, 1, 128)
             } else {
