@@ -198,12 +198,23 @@ PromptChunks prompt_chunks(int32_t T) { return PromptChunks{T / kAttnMaxTokens, 
 // form still serve up to 64 tokens (43 us over 2,048 rows of history). At head_dim 256 those launches take
 // 32-row chunks that each stream every key, and the prompt kernel is ahead from 33 tokens (24/4 heads, 64
 // tokens, 2,048 rows: 53 -> 33 us) until the history is so long that few row tiles cannot split it far
-// enough (33 tokens over 8,000 rows: 53 us by launches, 55 us here).
+// enough (33 tokens over 8,000 rows: 53 us by launches, 55 us here). That holds for more tokens over longer
+// histories, above all where the workspace leaves few splits (16/2 heads at head_dim 256, 200 tokens over 131,072
+// rows: 1,029 us by launches, 1,976 here; 24/4 over 32,768: 875 and 989; over 8,192: 366 and 263), so from 4,096 rows
+// the two are estimated. Of 612 measured calls eleven are 2 to 10% slower than the launches by that line (of the three
+// registered geometries one: 24/4 BF16, 320 tokens over 131,072 rows, 4%).
 bool prompt_kernel_serves(const AttnShape& s, const CacheRef& c, const nmi_tensor* q, const nmi_tensor* out,
-                          uint32_t max_keys) {
+                          uint32_t max_keys, size_t workspace_bytes, const PromptChunks& pc, const SplitPlan& full,
+                          const SplitPlan& last) {
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (c.kb == nullptr && !(aligned(c.kc) && aligned(c.vc) && aligned(c.ks) && aligned(c.vs))) { return false; }
-    return aligned(q->data) && aligned(out->data) && (s.T > 64 || (s.D == 256 && max_keys <= 4096));
+    if (!aligned(q->data) || !aligned(out->data)) { return false; }
+    if (max_keys <= 4096) { return s.T > 64 || s.D == 256; }
+    if (s.T <= 64) { return false; }
+    const bool bf16 = c.kb != nullptr;
+    const double launches = pc.full * verify_launch_us(full, s.Hkv, s.D, bf16, max_keys) +
+                            (pc.tail > 0 ? verify_launch_us(last, s.Hkv, s.D, bf16, max_keys) : 0.0);
+    return prompt_attention_us(s.T, s.Hq, s.Hkv, s.D, bf16, max_keys, workspace_bytes) <= launches;
 }
 
 // static_ws: the split partials go to the device's static scratch (the allocation-free entry
@@ -248,7 +259,7 @@ int attention_impl(const nmi_tensor* q, const nmi_tensor* k, const nmi_tensor* v
                 launch_kv_append(static_cast<const uint16_t*>(k->data), static_cast<const uint16_t*>(v->data),
                                  static_cast<const int32_t*>(positions->data), nullptr, CommitBounds{}, s.T, c, stream);
             }
-            if (prompt_kernel_serves(s, c, q, out, env.max_visible_keys)) {
+            if (prompt_kernel_serves(s, c, q, out, env.max_visible_keys, need, pc, full, last)) {
                 launch_prompt_attention(static_cast<const uint16_t*>(q->data), static_cast<const int32_t*>(positions->data),
                                         s.T, s.Hq, c, scale, env.max_visible_keys, ws, need, out->data, s.out_f32, stream);
                 return;

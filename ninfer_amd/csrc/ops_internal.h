@@ -104,6 +104,11 @@ void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uin
                              void* workspace, const SplitPlan& plan, void* out, bool out_f32,
                              hipStream_t stream);
 
+// Estimated times in us on MI355X, for the choice between the prompt kernel and verify launches: the
+// prompt kernel's over one call, and one verify launch's (with its merge).
+double prompt_attention_us(int32_t T, int32_t Hq, int32_t Hkv, int32_t D, bool bf16, uint32_t max_keys, size_t workspace_bytes);
+double verify_launch_us(const SplitPlan& plan, int32_t Hkv, int32_t D, bool bf16, uint32_t max_keys);
+
 // Causal attention of one sequence's T prompt tokens over cache rows that hold them already
 // (prompt_attention.hip). Key splits' partials go to the workspace, as many as fit.
 void launch_prompt_attention(const uint16_t* q, const int32_t* positions, int32_t T, int32_t Hq, const CacheRef& cache,

@@ -36,6 +36,7 @@
 #include "device_utils.h"
 #include "ops_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -1093,6 +1094,27 @@ PromptPlan plan_prompt(int32_t D, int64_t rows, int32_t Hkv, int32_t T, int64_t 
     return best;
 }
 
+// The time of plan_prompt's choice by the same model, for the choice between this kernel and verify launches:
+// constants fitted to 612 calls on MI355X (nine geometries, 65 to 1,024 tokens over 4,096 to 131,072 rows; 90% within
+// 14%).
+double plan_us(const PromptPlan& plan, int32_t D, bool bf16, int64_t rows, int32_t Hkv, int32_t T, int64_t max_keys) {
+    struct Fit {
+        double call, merge, tile[3]; // per key tile, by rows per workgroup: WK = 1, 2, 4
+        double far;                  // a tile's cost grows by this share up to a history of 131,072 rows
+    };
+    constexpr Fit fits[2][2] = {{{8.4, 3.4, {4.0, 2.35, 1.57}, 0.0}, {4.3, 5.3, {5.48, 3.36, 2.09}, 0.1}},
+                                {{9.3, 4.0, {2.42, 1.74, 0.0}, 0.02}, {8.9, 2.25, {3.04, 2.16, 0.0}, 0.08}}};
+    const Fit& f = fits[D == 128 ? 0 : 1][bf16 ? 1 : 0];
+    const double kt = 16384.0 / D;
+    const int64_t bm = (D == 128 ? 256 : 128) / plan.wk;
+    const double per_cu = static_cast<double>((rows + bm - 1) / bm * Hkv) * plan.nsplit / (kAttnTargetWorkgroups / 2);
+    const double longest = static_cast<double>(max_keys) / kt;
+    const double tiles = per_cu <= 1.0 ? longest : per_cu * (longest - 0.5 * T / kt) + 0.5 * longest;
+    return f.call + (plan.nsplit > 1 ? f.merge : 0.0) + 5.0 * std::max(per_cu, 1.0) +
+           f.tile[plan.wk == 1 ? 0 : plan.wk == 2 ? 1 : 2] * (1.0 + f.far * std::min(1.0, static_cast<double>(max_keys) / 131072.0)) * tiles /
+               plan.nsplit;
+}
+
 template <int D, bool BF>
 void launch_prompt(const PromptArgs& args, const PromptPlan& plan, void* workspace, hipStream_t stream) {
     PromptArgs a = args;
@@ -1122,6 +1144,11 @@ void launch_prompt(const PromptArgs& args, const PromptPlan& plan, void* workspa
 }
 
 } // namespace
+
+double prompt_attention_us(int32_t T, int32_t Hq, int32_t Hkv, int32_t D, bool bf16, uint32_t max_keys, size_t workspace_bytes) {
+    const int64_t rows = static_cast<int64_t>(T) * (Hq / Hkv);
+    return plan_us(plan_prompt(D, rows, Hkv, T, max_keys, workspace_bytes), D, bf16, rows, Hkv, T, max_keys);
+}
 
 void launch_prompt_attention(const uint16_t* q, const int32_t* positions, int32_t T, int32_t Hq, const CacheRef& c,
                              float scale, uint32_t max_keys, void* workspace, size_t workspace_bytes, void* out, bool out_f32,

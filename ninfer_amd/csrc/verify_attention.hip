@@ -2560,6 +2560,29 @@ size_t attention_workspace_bound(int32_t Hq, int32_t Hkv, int32_t D, int32_t T) 
     return bound;
 }
 
+// A batch-1 launch: its workgroups in rounds of the chip, each a split's keys long, or the keys' bytes where
+// they take longer. Constants fitted to the launches of the 612 prompts of prompt_attention_us (90% within 16%).
+double verify_launch_us(const SplitPlan& plan, int32_t Hkv, int32_t D, bool bf16, uint32_t max_keys) {
+    struct Fit {
+        double call, col;   // fixed, and per (row chunk, KV head)
+        double key, key_lone; // ns per key of a full round, and (two workgroups per CU) of one with at most one per CU
+        double bytes;         // TB/s
+    };
+    constexpr Fit fits[2][2] = {{{9.1, 0.19, 13.2, 7.3, 6.6}, {8.8, 0.25, 23.1, 8.8, 7.3}},
+                                {{13.1, 0.32, 17.6, 17.6, 6.35}, {13.4, 0.25, 18.4, 18.4, 7.2}}};
+    const Fit& f = fits[D == 128 ? 0 : 1][bf16 ? 1 : 0];
+    const int64_t cols = static_cast<int64_t>(Hkv) * plan.row_chunks;
+    const int64_t workgroups = cols * plan.nsplit;
+    constexpr int64_t cus = kAttnTargetWorkgroups / 2;
+    const bool wide = plan.rows_per_slot == kAttnWideRows;
+    const int64_t slots = D == 128 && !wide ? 2 * cus : cus;
+    const int64_t rest = workgroups % slots;
+    const double last = rest == 0 ? 0.0 : wide || rest <= cus ? f.key_lone : f.key;
+    const double keys = 1e-3 * plan.keys_per_split * (static_cast<double>(workgroups / slots) * (wide ? f.key_lone : f.key) + last);
+    const double row = Hkv * (bf16 ? 4.0 * D : 2.0 * D + D / 16.0); // K and V of one key
+    return f.call + f.col * static_cast<double>(cols) + std::max(keys, row * max_keys / (f.bytes * 1e6));
+}
+
 void launch_kv_append(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                       const int32_t* count, CommitBounds bounds, int32_t T, const CacheRef& c,
                       hipStream_t stream) {

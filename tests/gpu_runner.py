@@ -69,17 +69,25 @@ def run_attention(case, out_f32=False, mode="A1", cache=None, stream=None, envel
     return res, cache
 
 
-def attention_us(case) -> float:
-    """Device time of one A1 call."""
-    D, Hq, Hkv, T, B = case.D, case.Hq, case.Hkv, case.T, case.B
+def attention_us(case, tokens=None) -> float:
+    """Device time of the case's A1 calls: one call, or one per `tokens` tokens."""
+    D, Hq, Hkv, T = case.D, case.Hq, case.Hkv, case.T
     cache = upload_cache(case)
-    dev = [DeviceArray.from_numpy(na.BF16, case.q, (D, Hq, T, B)), DeviceArray.from_numpy(na.BF16, case.k_new, (D, Hkv, T, B)),
-           DeviceArray.from_numpy(na.BF16, case.v_new, (D, Hkv, T, B)), DeviceArray.from_numpy(na.I32, case.positions, (T, B))]
-    out = DeviceArray(na.BF16, (D, Hq, T, B))
-    env = (min(case.Ls) + T, case.max_context)
-    ws = DeviceBuffer(ops.gqa_attention_workspace_bytes(Hq, Hkv, D, T, B, env[1]))
-    views, view, o = [x.tensor() for x in dev], cache.view(), out.tensor()
-    return time_us(lambda: ops.gqa_attention(*views, case.scale, view, env, ws, o))
+    q, k, v = (DeviceArray.from_numpy(na.BF16, x) for x in (case.q, case.k_new, case.v_new))
+    pos, out = DeviceArray.from_numpy(na.I32, case.positions), DeviceArray(na.BF16, (D, Hq, T))
+    view, calls = cache.view(), []
+    for t0 in range(0, T, tokens or T):
+        n, end = min(tokens or T, T - t0), case.Ls[0] + min(t0 + (tokens or T), T)
+        qv, ov = (na.Tensor.make(x.ptr + 2 * D * Hq * t0, na.BF16, (D, Hq, n)) for x in (q, out))
+        kv, vv = (na.Tensor.make(x.ptr + 2 * D * Hkv * t0, na.BF16, (D, Hkv, n)) for x in (k, v))
+        calls.append((qv, kv, vv, na.Tensor.make(pos.ptr + 4 * t0, na.I32, (n,)), (end, end), ov))
+    ws = DeviceBuffer(max(ops.gqa_attention_workspace_bytes(Hq, Hkv, D, c[0].ne[2], 1, c[4][1]) for c in calls))
+
+    def run():
+        for qv, kv, vv, pv, env, ov in calls:
+            ops.gqa_attention(qv, kv, vv, pv, case.scale, view, env, ws, ov)
+
+    return time_us(run)
 
 
 def append(case, cache, stream=None):

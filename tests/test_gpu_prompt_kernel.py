@@ -143,6 +143,17 @@ def test_nan_key_is_not_dropped(gpu, L, T):
     assert not np.any(out[:, head])
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,kv,L,T", [(16, 2, 256, "i8", 65536, 96), (24, 4, 256, "bf16", 65536, 192), (40, 8, 128, "i8", 65536, 96),
+                                             (24, 4, 256, "i8", 16000, 128)])
+def test_long_history_cost(gpu, Hq, Hkv, D, kv, L, T):
+    """A prompt over a long history takes no longer than the same tokens in calls of 32 (10% for the estimates
+    that choose the route; MI355X: 0.5 to 1.0, where the prompt kernel alone took up to 2)."""
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, kv=kv, seed=2, gen="pcg")
+    whole, parts = gpu_runner.attention_us(case), gpu_runner.attention_us(case, tokens=32)
+    print(f"{Hq}/{Hkv}/{D} {kv} L={L} T={T}: {whole:.1f} us, in calls of 32 {parts:.1f} us")
+    assert whole <= 1.1 * parts
+
+
 def test_unaligned_tensors_take_the_verify_launches(gpu):
     """q one element into its buffer: accepted as before, and within the same bar."""
     case = AttnCase([200], T=70, seed=17)
