@@ -116,10 +116,25 @@ __device__ __forceinline__ void stage_load(const GdnArgs& a, int t0, int h, int 
     r.beta = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(chunk_rows(a.beta, 4 * a.Hv, t0, a.T), past, 0, 0));
 }
 
-// Fills chunk c (one wave).
-__device__ __forceinline__ void stage_store(const GdnArgs& a, const Stage& r, Chunk& x, int lane) {
-    const int c = lane & 15;
-    const int g = lane >> 4;
+// Zeros the staged rows of v whose factors are 0: a squared norm beyond FP32. Their normalized row is 0 where every value
+// is finite; a row with an infinite value stays as it is (0 x inf is NaN in its products, as it is in the row).
+__device__ __forceinline__ void drop_overflowed(w4 (&v)[2][4], const float* factors, int lane) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int quad = (lane + 64 * u) >> 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { bad |= (((v[u][e][i] & 0x7f807f80u) + 0x00800080u) & 0x80008000u) != 0u; }
+            const uint64_t row = (__ballot(bad) >> (lane & 48)) & 0xffffu; // 16 lanes hold a row
+            if (factors[4 * quad + e] == 0.0f && row == 0u) { v[u][e] = w4{0u, 0u, 0u, 0u}; }
+        }
+    }
+}
+
+// The rows of k and q and the columns of k^T of chunk x, from the staging wave's registers.
+__device__ __forceinline__ void stage_rows(const Stage& r, Chunk& x, int lane) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int unit = lane + 64 * u;
@@ -145,7 +160,11 @@ __device__ __forceinline__ void stage_store(const GdnArgs& a, const Stage& r, Ch
             *reinterpret_cast<w2*>(x.kt + kt_at(8 * oct + i, quad & 3) + 8 * (quad >> 2)) = p;
         }
     }
-    // the wave's own LDS writes above are complete before its reads below (in-order LDS)
+}
+
+// Products of the chunk's tokens: [token tile][i tile], row 4g + e, column c. The wave's own LDS writes are complete
+// before these reads (in-order LDS).
+__device__ __forceinline__ void stage_products(const Chunk& x, int c, int g, f4 (&kk)[2][2], f4 (&qk)[2][2], f4 (&qq)[2]) {
     b8 kr[2][4], qr[2][4];
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
@@ -156,7 +175,6 @@ __device__ __forceinline__ void stage_store(const GdnArgs& a, const Stage& r, Ch
         }
     }
     const f4 zero = {0.f, 0.f, 0.f, 0.f};
-    f4 kk[2][2], qk[2][2], qq[2]; // [token tile][i tile]: row 4g + e, column c
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
 #pragma unroll
@@ -173,16 +191,41 @@ __device__ __forceinline__ void stage_store(const GdnArgs& a, const Stage& r, Ch
 #pragma unroll
         for (int s = 0; s < 4; ++s) { qq[tt] = mfma_b(qr[tt][s], qr[tt][s], qq[tt]); }
     }
-    // per-token factors through LDS: the squared norms sit on the diagonals (lane (c, c / 4), entry c % 4)
+}
+
+// Per-token factors to x.gk and x.gq: the squared norms sit on the diagonals (lane (c, c / 4), entry c % 4). Returns
+// whether a factor is 0.
+__device__ __forceinline__ bool stage_factors(bool normalize, const f4 (&kk)[2][2], const f4 (&qq)[2], Chunk& x, int c, int g) {
+    bool none = false;
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
         const float nk = (c & 2) ? ((c & 1) ? kk[tt][tt][3] : kk[tt][tt][2]) : ((c & 1) ? kk[tt][tt][1] : kk[tt][tt][0]);
         const float nq = (c & 2) ? ((c & 1) ? qq[tt][3] : qq[tt][2]) : ((c & 1) ? qq[tt][1] : qq[tt][0]);
         if (g == (c >> 2)) {
             // x / sqrt(sum(x^2) + 1e-6) over the row (gated_delta_rule.h:35-36)
-            x.gk[16 * tt + c] = a.normalize_qk ? 1.0f / sqrtf(nk + 1.0e-6f) : 1.0f;
-            x.gq[16 * tt + c] = a.normalize_qk ? 1.0f / sqrtf(nq + 1.0e-6f) : 1.0f;
+            const float fk = normalize ? 1.0f / sqrtf(nk + 1.0e-6f) : 1.0f;
+            const float fq = normalize ? 1.0f / sqrtf(nq + 1.0e-6f) : 1.0f;
+            x.gk[16 * tt + c] = fk;
+            x.gq[16 * tt + c] = fq;
+            none |= fk == 0.0f || fq == 0.0f;
         }
+    }
+    return none;
+}
+
+// Fills chunk x (one wave).
+__device__ __forceinline__ void stage_store(const GdnArgs& a, Stage& r, Chunk& x, int lane) {
+    const int c = lane & 15;
+    const int g = lane >> 4;
+    f4 kk[2][2], qk[2][2], qq[2];
+    stage_rows(r, x, lane);
+    stage_products(x, c, g, kk, qk, qq);
+    if (__builtin_expect(__any(stage_factors(a.normalize_qk != 0, kk, qq, x, c, g)), 0)) {
+        drop_overflowed(r.k, x.gk, lane);
+        drop_overflowed(r.q, x.gq, lane);
+        stage_rows(r, x, lane);
+        stage_products(x, c, g, kk, qk, qq);
+        (void)stage_factors(a.normalize_qk != 0, kk, qq, x, c, g);
     }
     // decays as exp of differences of the running sum of g in 64 bits (beyond +-1000 exp(g) is 0 or
     // infinite either way; a NaN stays)

@@ -62,6 +62,25 @@ def test_non_finite_token_leaves_earlier_outputs(gpu, where):
     assert np.isnan(out[40]).any()
 
 
+@pytest.mark.parametrize("rows", [[(20, "k")], [(33, "q")], [(5, "k"), (40, "k"), (40, "q"), (65, "q")]])
+def test_squared_norm_beyond_fp32(gpu, rows):
+    """A finite k or q row whose squared norm overflows FP32 is normalized to 0, as token by token: the token decays
+    the state and adds nothing, or puts out 0, and no other token sees it."""
+    T, H = 66, 3
+    inp = _inputs(78, 128, H, H, T, normalized=False)
+    zeroed = {n: x.copy() for n, x in inp.items()}
+    for t, n in rows:
+        inp[n].reshape(T, H, 128)[t, 1, ::3] = _bf(np.array([3.0e38], np.float32))[0]
+        zeroed[n].reshape(T, H, 128)[t, 1] = 0
+    ref_out, ref_state = _oracle(zeroed, H, H, T, True)[:2]
+    out, state = run_regular(inp, 128, H, H, T, True, False)
+    _ok(_f(out).reshape(T, H, 128), ref_out, GDN_OUTPUT_BF16, "out")
+    assert np.linalg.norm(state - ref_state) / np.linalg.norm(ref_state) <= STATE_REL
+    head = {n: x if n == "state" else np.ascontiguousarray(x.reshape(T, -1)[:16]).reshape(16, *x.shape[1:]) for n, x in inp.items()}
+    first, _ = run_regular(head, 128, H, H, 16, True, False)
+    _ok(_f(out).reshape(T, H, 128)[:16], _f(first).reshape(16, H, 128), GDN_OUTPUT_BF16, "token by token")
+
+
 @pytest.mark.parametrize("C,T,offset,in_place", [(10240, 17, 0, False), (10240, 1700, 0, True), (1001, 33, 0, True), (64, 16, 0, False),
                                                  (130, 100, 0, False), (512, 40, 1, True), (24, 19, 0, True)])
 def test_conv_prompt(gpu, C, T, offset, in_place):
