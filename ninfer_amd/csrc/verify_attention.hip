@@ -2359,25 +2359,27 @@ __global__ __launch_bounds__(256) void kv_quant_append_kernel(const uint16_t* k,
     }
 }
 
-// Column (t, b), KV head and 8-element piece of a flat index over k/v [D, Hkv, T, B] (source offset
-// 8u), and the cache row of the column (-1: the column is not written).
+// Column (t, b), KV head and 8-element piece of a flat index over the columns of k/v [D, Hkv, T, B] from col0
+// (source offset 8u), and the cache row of the column (-1: the column is not written).
 struct AppendUnit {
     int piece, h, b, row;
 };
 
-__device__ __forceinline__ AppendUnit append_unit(uint32_t u, uint32_t pieces, const int32_t* positions, const int32_t* count,
-                                                  CommitBounds cb, int32_t T, int32_t Hkv, int32_t P) {
+__device__ __forceinline__ AppendUnit append_unit(uint32_t u, uint32_t pieces, uint32_t col0, const int32_t* positions,
+                                                  const int32_t* count, CommitBounds cb, int32_t T, int32_t Hkv, int32_t P) {
     AppendUnit x;
     const uint32_t th = u / pieces;
     x.piece = static_cast<int>(u - th * pieces);
-    const int col = static_cast<int>(th / static_cast<uint32_t>(Hkv));
-    x.h = static_cast<int>(th - static_cast<uint32_t>(col) * static_cast<uint32_t>(Hkv));
-    x.b = col / T;
+    const uint32_t c = th / static_cast<uint32_t>(Hkv);
+    x.h = static_cast<int>(th - c * static_cast<uint32_t>(Hkv));
+    const uint32_t col = col0 + c;
+    const uint32_t b = col / static_cast<uint32_t>(T);
+    x.b = static_cast<int>(b);
     const int p = positions[col];
     x.row = p < 0 || (p & cb.slot_mask) >= P ? -1 : p & cb.slot_mask;
     if (count != nullptr) {
         const int n = count[x.b];
-        if (n < cb.min_count || n > cb.max_count || col - x.b * T >= n) { x.row = -1; }
+        if (n < cb.min_count || n > cb.max_count || static_cast<int>(col - b * static_cast<uint32_t>(T)) >= n) { x.row = -1; }
     }
     return x;
 }
@@ -2390,11 +2392,11 @@ template <int D>
 __global__ __launch_bounds__(256) void kv_quant_append_rows_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                                                                    const int32_t* count, CommitBounds cb, int32_t T, int32_t Hkv,
                                                                    int32_t P, int8_t* kc, int8_t* vc, uint16_t* ks, uint16_t* vs,
-                                                                   int64_t code_seq, int64_t scale_seq, uint32_t units) {
+                                                                   int64_t code_seq, int64_t scale_seq, uint32_t col0, uint32_t units) {
     const uint32_t u = blockIdx.x * 256 + threadIdx.x;
     if (u >= units) { return; } // units is a multiple of 8: whole groups stay together
     const i4 raw = *reinterpret_cast<const i4*>((blockIdx.y ? v : k) + static_cast<int64_t>(u) * 8);
-    const AppendUnit a = append_unit(u, D / 8, positions, count, cb, T, Hkv, P);
+    const AppendUnit a = append_unit(u, D / 8, col0, positions, count, cb, T, Hkv, P);
     float x[8];
     float amax = 0.0f;
 #pragma unroll
@@ -2432,11 +2434,11 @@ __global__ __launch_bounds__(256) void kv_quant_append_rows_kernel(const uint16_
 __global__ __launch_bounds__(256) void bf16_kv_append_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                                                              const int32_t* count, CommitBounds cb, int32_t T,
                                                              int32_t Hkv, int32_t P, int32_t D, uint16_t* kb,
-                                                             uint16_t* vb, int64_t seq, uint32_t units) {
+                                                             uint16_t* vb, int64_t seq, uint32_t col0, uint32_t units) {
     const uint32_t u = blockIdx.x * 256 + threadIdx.x;
     if (u >= units) { return; }
     const i4 raw = *reinterpret_cast<const i4*>((blockIdx.y ? v : k) + static_cast<int64_t>(u) * 8);
-    const AppendUnit a = append_unit(u, D / 8, positions, count, cb, T, Hkv, P);
+    const AppendUnit a = append_unit(u, D / 8, col0, positions, count, cb, T, Hkv, P);
     if (a.row < 0) { return; }
     uint16_t* dst = (blockIdx.y ? vb : kb) + static_cast<int64_t>(a.b) * seq + static_cast<int64_t>(D) * (a.row + static_cast<int64_t>(P) * a.h);
     *reinterpret_cast<i4*>(dst + 8 * a.piece) = raw;
@@ -2586,18 +2588,9 @@ double verify_launch_us(const SplitPlan& plan, int32_t Hkv, int32_t D, bool bf16
 void launch_kv_append(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                       const int32_t* count, CommitBounds bounds, int32_t T, const CacheRef& c,
                       hipStream_t stream) {
-    const int64_t units = static_cast<int64_t>(T) * c.B * c.Hkv * (c.D / 8); // 8-element pieces of k
-    if (units > 0xffffff00) { throw Unsupported("kv append: 2^35 or more elements in one call are not built"); }
-    const dim3 flat(static_cast<unsigned>((units + 255) / 256), 2);
-    if (c.kb != nullptr) {
-        hipLaunchKernelGGL(bf16_kv_append_kernel, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T, c.Hkv,
-                           c.P, c.D, c.kb, c.vb, c.code_seq, static_cast<uint32_t>(units));
-        check_launch("bf16_kv_append_kernel");
-        return;
-    }
     const auto misaligned = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
-    if (c.D != 128 && c.D != 256) { throw Unsupported("kv append: head_dim 128 and 256 are built"); }
-    if (misaligned(k, 16) || misaligned(v, 16) || misaligned(c.kc, 8) || misaligned(c.vc, 8)) {
+    if (c.kb == nullptr && c.D != 128 && c.D != 256) { throw Unsupported("kv append: head_dim 128 and 256 are built"); }
+    if (c.kb == nullptr && (misaligned(k, 16) || misaligned(v, 16) || misaligned(c.kc, 8) || misaligned(c.vc, 8))) {
         // 2-byte loads and 1-byte stores for tensors the wide form cannot address
         const dim3 grid(T, c.B, c.Hkv);
         if (c.D == 128) {
@@ -2607,14 +2600,31 @@ void launch_kv_append(const uint16_t* k, const uint16_t* v, const int32_t* posit
             hipLaunchKernelGGL(kv_quant_append_kernel<256>, grid, dim3(256), 0, stream, k, v, positions,
                                count, bounds, T, c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq);
         }
-    } else if (c.D == 128) {
-        hipLaunchKernelGGL(kv_quant_append_rows_kernel<128>, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T,
-                           c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, static_cast<uint32_t>(units));
-    } else {
-        hipLaunchKernelGGL(kv_quant_append_rows_kernel<256>, flat, dim3(256), 0, stream, k, v, positions, count, bounds, T,
-                           c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, static_cast<uint32_t>(units));
+        check_launch("kv_quant_append_kernel");
+        return;
     }
-    check_launch("kv_quant_append_kernel");
+    // 8-element pieces of whole columns, as many as a grid of 2^32 threads holds (one launch below 2^35 elements)
+    const int64_t per_col = static_cast<int64_t>(c.Hkv) * (c.D / 8);
+    const int64_t columns = static_cast<int64_t>(T) * c.B;
+    const int64_t most = std::max<int64_t>(1, 0xffffff00 / per_col);
+    for (int64_t col0 = 0; col0 < columns; col0 += most) {
+        const uint32_t units = static_cast<uint32_t>(std::min(most, columns - col0) * per_col);
+        const dim3 flat(static_cast<unsigned>((static_cast<uint64_t>(units) + 255) / 256), 2);
+        const uint16_t* kc0 = k + col0 * per_col * 8;
+        const uint16_t* vc0 = v + col0 * per_col * 8;
+        const uint32_t first = static_cast<uint32_t>(col0);
+        if (c.kb != nullptr) {
+            hipLaunchKernelGGL(bf16_kv_append_kernel, flat, dim3(256), 0, stream, kc0, vc0, positions, count, bounds, T, c.Hkv,
+                               c.P, c.D, c.kb, c.vb, c.code_seq, first, units);
+        } else if (c.D == 128) {
+            hipLaunchKernelGGL(kv_quant_append_rows_kernel<128>, flat, dim3(256), 0, stream, kc0, vc0, positions, count, bounds, T,
+                               c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, first, units);
+        } else {
+            hipLaunchKernelGGL(kv_quant_append_rows_kernel<256>, flat, dim3(256), 0, stream, kc0, vc0, positions, count, bounds, T,
+                               c.Hkv, c.P, c.kc, c.vc, c.ks, c.vs, c.code_seq, c.scale_seq, first, units);
+        }
+        check_launch("kv_append_kernel");
+    }
 }
 
 void launch_verify_attention(const uint16_t* q, const uint16_t* k_new, const uint16_t* v_new,

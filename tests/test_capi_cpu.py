@@ -11,7 +11,7 @@ import pytest
 
 import ninfer_amd as na
 from ninfer_amd import ops
-from ninfer_amd._capi import INVALID_ARGUMENT, Tensor, lib
+from ninfer_amd._capi import INVALID_ARGUMENT, NmiError, Tensor, lib
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -549,3 +549,18 @@ def test_runtime_helper_validation():
     assert L.nmi_rt_next_row_i32(None, 4, 3, fake, fake, None) == INVALID_ARGUMENT
     assert L.nmi_rt_next_row_i32(fake, 0, 3, fake, fake, None) == INVALID_ARGUMENT
     assert L.nmi_rt_next_row_i32(fake, 4, 1025, fake, fake, None) == INVALID_ARGUMENT
+
+
+def test_append_has_no_limit_on_elements():
+    """2^35 elements and more reach the launch (no GPU here: a HIP error), as any smaller call."""
+    from ninfer_amd import device
+    try:
+        present = device.device_count() > 0
+    except NmiError:
+        present = False
+    if present:
+        pytest.skip("launches: the addresses are not real")
+    T, B = 1 << 20, 32
+    k, pos, count = _t(na.BF16, (128, 8, T, B)), _t(na.I32, (T, B)), _t(na.I32, (B,))
+    with pytest.raises(NmiError):
+        ops.kv_cache_append_prefix(k, k, pos, count, (0, 100), _cache(B=B))

@@ -197,3 +197,32 @@ def test_append_forms(gpu, D, T, B, offset):
     synchronize()
     for got, want in zip(cache.download(), (kc, vc, ks, vs)):
         assert np.array_equal(got, want)
+
+
+def test_append_of_several_launches(gpu):
+    """2^35 elements of K: more 8-element pieces than one grid holds. Two columns of each of 32 sequences are
+    committed, the last ones' by the second launch, with the oracle's codes."""
+    from oracle import pyoracle
+    T, B, Hkv, D, P, n = 1 << 20, 32, 8, 128, 256, 2
+    row = Hkv * D
+    src = DeviceArray(na.BF16, (D, Hkv, T, B))  # 64 GiB, only the committed columns written
+    rng = np.random.default_rng(12)
+    cols = (rng.normal(size=(B, n, row)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    for b in range(B):
+        src.buf.upload(cols[b], 2 * row * T * b)
+    positions = np.full((B, T), -1, np.int32)
+    positions[:, :n] = np.arange(B)[:, None] * 2 + np.arange(n)
+    pos = DeviceArray.from_numpy(na.I32, positions, (T, B))
+    count = DeviceArray.from_numpy(na.I32, np.full(B, n, np.int32), (B,))
+    from ninfer_amd.kv_cache import KVCacheLayer
+    cache = KVCacheLayer(P, Hkv, D, B)
+    planes = [np.zeros((B, Hkv, P, D), np.int8), np.zeros((B, Hkv, P, D), np.int8),
+              np.zeros((B, Hkv, P, D // 64), np.uint16), np.zeros((B, Hkv, P, D // 64), np.uint16)]
+    cache.upload(*planes)
+    ops.kv_cache_append_prefix(src.tensor(), src.tensor(), pos.tensor(), count.tensor(), (0, n), cache.view())
+    synchronize()
+    for b in range(B):
+        one = cols[b].reshape(-1)
+        pyoracle.kv_append(one, one, positions[b, :n].copy(), n, 1, Hkv, D, P, *(x[b] for x in planes))
+    for got, want in zip(cache.download(), planes):
+        assert np.array_equal(got.reshape(want.shape), want)
