@@ -49,6 +49,48 @@ def test_wide_envelope(gpu, L, T, cap):
     _run(case, envelope=(1, cap))
 
 
+def _attend64(case, planes, last):
+    """Attention in 64 bits of every token over the cache rows [0, last]."""
+    f32 = lambda bits: (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)  # noqa: E731
+    if case.kv == "bf16":
+        k, v = (f32(x[0]) for x in planes)
+    else:
+        k, v = (c[0].astype(np.float64) * np.repeat(s[0].view(np.float16).astype(np.float64), 64, axis=-1)
+                for c, s in ((planes[0], planes[2]), (planes[1], planes[3])))
+    n = int(last.max()) + 1
+    q = f32(case.q).reshape(case.T, case.Hkv, -1, case.D)
+    hidden = np.arange(n)[None, :] > last[:, None]
+    out = np.empty(q.shape)
+    for h in range(case.Hkv):
+        score = np.einsum("tgd,kd->tgk", q[:, h], k[h, :n], optimize=True) * case.scale
+        score[np.broadcast_to(hidden[:, None], score.shape)] = -np.inf
+        p = np.exp(score - score.max(-1, keepdims=True))
+        out[:, h] = np.einsum("tgk,kd->tgd", p / p.sum(-1, keepdims=True), v[h, :n], optimize=True)
+    return out.reshape(-1)
+
+
+# An envelope that ends before the last positions: a token sees the keys up to its position or the envelope's end.
+@pytest.mark.parametrize("Hq,Hkv,D,kv,L,T,cap", [
+    (40, 8, 128, "i8", 100, 300, 350), (40, 8, 128, "i8", 2500, 80, 2530), (40, 8, 128, "i8", 100, 200, 200), (24, 4, 256, "i8", 30, 300, 301),
+    (16, 2, 256, "bf16", 1500, 70, 1510), (40, 8, 128, "bf16", 100, 1000, 1003)])
+@pytest.mark.parametrize("rare", [False, True])
+def test_envelope_clamps_positions(gpu, Hq, Hkv, D, kv, L, T, cap, rare):
+    if rare and kv == "bf16":
+        pytest.skip("scales are INT8's")
+    print(f"case prompt clamp {Hq}/{Hkv}/{D} {kv} L={L} T={T} cap={cap} rare={rare}", flush=True)
+    case = AttnCase([L], T=T, Hq=Hq, Hkv=Hkv, D=D, kv=kv, seed=41, qstd=2e-5 if rare else 1.0)
+    if rare:
+        _rare_scales(case, 3)
+    planes, _ = case.oracle_after_append()
+    ref = _attend64(case, planes, np.minimum(case.positions, cap - 1))
+    out, cache = gpu_runner.run_attention(case, out_f32=True, envelope=(1, cap))
+    for got, want in zip(cache.download(), planes):
+        assert np.array_equal(got, want)
+    err = rel_l2(out, ref)
+    print(f"rel_l2={err:.3e}", flush=True)
+    assert np.all(np.isfinite(out)) and err <= REL_L2_F32
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,L,T", [(40, 8, 128, 100, 65), (40, 8, 128, 2600, 65), (24, 4, 256, 150, 40), (24, 4, 256, 1500, 40)])
 @pytest.mark.parametrize("absmax", [1e5, 1e6])
 def test_fp32_range(gpu, Hq, Hkv, D, L, T, absmax):
