@@ -171,7 +171,8 @@ int nmi_gqa_attention_workspace_bound(int32_t q_heads, int32_t tokens, size_t* b
  * out may also be FP32 (EXTENSION). T above 32 is the reference's prompt route
  * (src/ops/wrapper/gqa_attention.cpp:202-213): one sequence (B = 1); the rows are appended first,
  * then the tokens attend through the same workspace: in one prompt kernel (and a merge where it splits the
- * keys), or in verify launches of 32 for short prompts and for q, out or cache planes off 16 bytes. */
+ * keys), or in verify launches of 32 for short prompts, for long histories over which the launches are faster, and
+ * for q, out or cache planes off 16 bytes. */
 int nmi_gqa_attention(const nmi_tensor* q, const nmi_tensor* k, const nmi_tensor* v,
                       const nmi_tensor* positions, float scale, const nmi_kv_layer_view* cache,
                       nmi_gqa_envelope envelope, void* workspace, size_t workspace_bytes,

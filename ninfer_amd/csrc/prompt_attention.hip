@@ -15,8 +15,8 @@
 //    writes nor the operand reads conflict) and tile j is multiplied. One barrier per tile.
 //  * S^T = K' Q^T and O^T = V'^T P^T on 16x16x32 MFMAs, as in verify_attention.hip: the S^T
 //    accumulator layout is the P^T operand layout (the V^T key order inside 32 keys follows it), so
-//    probabilities stay in registers. Same operand roundings and lazy softmax as the verify kernels;
-//    a tile's rows see all keys in one workgroup, so no FP16 partials are written at all.
+//    probabilities stay in registers. Same operand roundings and lazy softmax as the verify kernels; a
+//    tile's rows see all keys in one workgroup, so no FP16 partials are written unless the keys are split.
 //  * WK waves share a row tile and take different 32-key chunks of each key tile (merged through
 //    LDS at the end), so that short prompts still give every CU rows of its own.
 //  * A prompt with too few row tiles for the chip also splits the keys over workgroups (FP16 O / l
@@ -25,12 +25,13 @@
 //    keeps few heads' keys in its L2.
 //
 // Measured on MI355X (A1, append included) against the verify launches of 32 tokens: 2,048 tokens over
-// 2,048 rows at 40/8/128 1,405 -> 188 us (685 TFLOP/s of the causal products; 8,192 tokens 920, where a
-// large library product reaches 1,180), BF16 cache 1,803 -> 235 us; 1,000 tokens at 24/4/256 760 -> 49
-// us; 65 tokens over 2,048 rows 53 -> 26 us. What is left: MFMA is busy 41% and the VALU (decode,
-// exponentials) 53% of the SIMD time and the two hardly overlap; issuing the next chunk's S^T under
-// the exponentials (833), alternating the wave halves by barriers (842) and raised issue priority
-// (911) were no better than the plain order (919 TFLOP/s at 8,192 tokens).
+// 2,048 rows at 40/8/128 1,403 -> 187 us (689 TFLOP/s of the causal products; 8,192 tokens 916, where a
+// large library product reaches 1,180), BF16 cache 1,804 -> 243 us; 1,000 tokens at 24/4/256 758 -> 46
+// us; 65 tokens over 2,048 rows 51 -> 23 us. What is left at 2,048 tokens: MFMA is busy 42% and the VALU
+// (decode, exponentials) 57% of the SIMD time (profiles/prompts_and_column_acceptance.txt) and the two hardly
+// overlap; issuing the next chunk's S^T under the exponentials (833), alternating the wave halves by
+// barriers (842) and raised issue priority (911) were no better than the plain order (919 TFLOP/s at 8,192
+// tokens, all four in one build).
 #include "attn_math.h"
 #include "common.h"
 #include "device_utils.h"

@@ -2386,8 +2386,8 @@ __device__ __forceinline__ AppendUnit append_unit(uint32_t u, uint32_t pieces, u
 
 // The same encoder over 16-byte aligned k/v and 8-byte aligned code planes: a lane owns 8 consecutive
 // elements, 8 lanes a group, so a wave reads 1 KB and writes 512 B whole. Launch-bound for a verify
-// round's few rows; a 2,048-token prompt of 8 heads (34 MB read and written) took 13.5 us with a wave
-// per 64-element group in 16,384 workgroups of 2-byte loads and 6.4 us this way. y: K or V.
+// round's few rows; a 2,048-token prompt of 8 heads (13 MB read and written) took 13.5 us with a wave
+// per 64-element group in 16,384 workgroups of 2-byte loads and takes 6.0 us this way (kernel time). y: K or V.
 template <int D>
 __global__ __launch_bounds__(256) void kv_quant_append_rows_kernel(const uint16_t* k, const uint16_t* v, const int32_t* positions,
                                                                    const int32_t* count, CommitBounds cb, int32_t T, int32_t Hkv,
