@@ -452,7 +452,8 @@ constexpr uint32_t kOrderedInf = 0xff80u, kOrderedNegInf = 0x007fu; // ordered16
 constexpr int kHot = 128;        // most frequent values counted apart
 constexpr int kHotLanes = 32;    // counters of one (lane l and l + 32 share one)
 constexpr uint32_t kHotAt = 8;   // of 1,024 sampled tokens: a value counts as frequent
-constexpr uint32_t kHotOne = 80; // one value this frequent, or kHotFew frequent ones: they are counted apart
+constexpr uint32_t kHotOne = 80; // one value this frequent (half of what a counter holds, in long columns), or kHotFew
+                                 // frequent ones: they are counted apart
 constexpr uint32_t kHotFew = 24;
 constexpr int kTags = 1024;
 constexpr int kAhead = 8;        // 16-byte loads in flight per thread in a walk
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(kColThreads) void gen_column_kernel(GenArgs a) {
             const uint32_t slot = atomicAdd(&hot_n, 1u);
             if (slot < kHot) { hot_bits[slot] = sample; }
         }
-        if (seen == kHotOne - 1) { hot_top = 1u; }
+        if (seen == min(kHotOne, kColThreads * 32768u / static_cast<uint32_t>(a.V)) - 1u) { hot_top = 1u; }
         __syncthreads();
     }
     const bool few = hot_top != 0u || hot_n >= kHotFew;

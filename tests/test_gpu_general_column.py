@@ -32,6 +32,11 @@ def _columns(kind, t, d):
         elif kind == "fifty_values":  # more frequent values than are counted apart, sharing hash buckets or not
             vals = rng.permutation(np.r_[0x3C00:0x4080, 0xBC00:0xC080])[:50].astype(np.uint16)
             x[:] = vals[rng.integers(0, 50, x.shape)]
+        elif kind == "wraps":  # a value that overflows its counter and is at none of the 1,024 sampled places
+            rows, bits = x.shape[-1], 0x4049 if x is t else 0xBFC1
+            common = rng.random(x.shape, dtype=np.float32) < 0.1
+            common[..., np.arange(1024) * rows // 1024] = False
+            x[common] = bits
         elif kind == "constant":
             x[:] = 0x3E4D
         elif kind == "nan":
@@ -55,6 +60,7 @@ def _columns(kind, t, d):
     ("masked_integers", 10, 3, 150000, 0.7, 0.9),
     ("fifty_values", 10, 3, 100000, 1.0, 0.4),
     ("constant", 10, 3, 65552, 0.7, 0.5),
+    ("wraps", 22, 1, 700001, 0.7, 0.9),
 ])
 def test_column_route(gpu, oracle, kind, B, K, rows, temp, top_p):
     t, d, dr, ua, ur = _case(60 + rows % 17, B, K, rows)
